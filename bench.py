@@ -82,6 +82,16 @@ KERNELS = {
              "dct_inv": "k_fdct_inv<double, 8>", "phi_inv": "k_fphi_inv<double, 8, 512, false>"},
 }
 
+
+def dense_fp64(form, bw, nfields):
+    """The FP64 call runs the dense Legendre GEMMs (s2_naive64.hip) and no DCT stage."""
+    return form == "fp64" and 16 <= bw <= 512 and (bw <= 320 or nfields >= 4)
+
+
+def legendre_form(form, bw, nfields):
+    """`form`, or "mixed" for an FP64 call on the dense GEMMs: the naive transform's stages, bytes and flops."""
+    return "mixed" if dense_fp64(form, bw, nfields) else form
+
 def smooth(n, pmax):
     """n has no prime factor above pmax."""
     for p in range(2, pmax + 1):
@@ -122,14 +132,25 @@ def kernels_gen(bw, form):
 
 def kernel_map(form, bw, nfields):
     """Kernel behind each timed stage of a batched call of nfields fields on
-    an all-seminaive plan.  The FP64/FP32 GEMMs run K-chunked (64 columns per
+    an all-seminaive plan.  The FP32 GEMMs run K-chunked (64 columns per
     block; 512 threads up to bw = 256, 1024 above) at bw in [128, 512] with 64
-    or more fields."""
+    or more fields; so do the dense FP64 ones (the inverse always 512
+    threads), above bw = 256 from 16 fields, and with 32 columns per block
+    (negative last argument in the forward) from bw^2 x fields = 300000."""
     k = dict(KERNELS[form] if bw & (bw - 1) == 0 else kernels_gen(bw, form))
-    if form in ("fp64", "fp32") and 128 <= bw <= 512 and nfields >= 64:
-        r = "double" if form == "fp64" else "float"
+    if dense_fp64(form, bw, nfields):
+        k.pop("dct_fwd"), k.pop("dct_inv")
+        h = 1 if bw <= 256 else 2
+        if bw >= 128 and nfields * bw * bw >= 300000:
+            if nfields >= 64 or (h == 2 and nfields >= 16):
+                k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd_kc<double, {512 * h}>", "k_gemm_inv_kc<double, 512>"
+            else:
+                k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd<double, false, 2, {-h}>", "k_gemm_inv_kc<double, 256>"
+        else:
+            k["leg_fwd"], k["leg_inv"] = "k_gemm_fwd<double, false, CT", "k_gemm_inv<double, false, CT"
+    elif form == "fp32" and 128 <= bw <= 512 and nfields >= 64:
         t = 512 if bw <= 256 else 1024
-        k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd_kc<{r}, {t}>", f"k_gemm_inv_kc<{r}, {t}>"
+        k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd_kc<float, {t}>", f"k_gemm_inv_kc<float, {t}>"
     return k
 
 
@@ -695,7 +716,8 @@ def main():
     dom = max(stages, key=lambda k: stages[k][0])
     dom_ms, dom_n = stages[dom]
     avg_s = dom_ms / dom_n / 1e3
-    achieved = stage_bytes(dom, bw, F, elem, args.precision) / avg_s
+    lform = legendre_form(args.precision, bw, F)
+    achieved = stage_bytes(dom, bw, F, elem, lform) / avg_s
     roofline = {
         "bound": "hbm",
         "kernel": kernel_map(args.precision, bw, F).get(dom, dom),
@@ -705,7 +727,7 @@ def main():
         "unit": "GB/s",
         "frac": achieved / HBM_PEAK,
         "traffic": measured_traffic(args.precision, bw, F, dom),
-        "algorithmic_bytes": stage_bytes(dom, bw, F, elem, args.precision),
+        "algorithmic_bytes": stage_bytes(dom, bw, F, elem, lform),
         "avg_launch_ms": dom_ms / dom_n,
         "stages_ms_per_step": {k: v[0] / args.steps for k, v in stages.items()},
     }
@@ -717,7 +739,7 @@ def main():
     for st_ in ("leg_fwd", "leg_inv"):
         if st_ in stages:
             ms, cnt = stages[st_]
-            useful = legendre_flops(bw, F, args.precision) / (ms / cnt / 1e3) / 1e12
+            useful = legendre_flops(bw, F, lform) / (ms / cnt / 1e3) / 1e12
             # the seminaive count (cosine-series table MACs) is the transform's
             # algorithmic work whatever the form; the naive forms do 4 bw^3 per
             # field instead, more MACs for the same coefficients

@@ -350,6 +350,8 @@ struct Plan {
     DevConsts c;
     DevTables t;
     GemmTables g;
+    GemmTables gd;  // FP64, bw <= 512: dense tables (s2_naive64.hip), for calls of dense_min fields or more
+    int dense_min = 0;  // 0: none
     DBuf X, Cb, cr, ci, zr, zi;
     StageTimer timer;
 };
@@ -365,6 +367,9 @@ static bool use_fast(const Plan* p, int F) {
     return F >= 2 || p->bw < 512;
 }
 
+// The GEMM tables of a call of F fields.
+static GemmTables& gemm_of(Plan* p, int F) { return p->dense_min && F >= p->dense_min ? p->gd : p->g; }
+
 // The forward pipeline of a plan on scratch X (order-major intermediate) and
 // Cb (cosine rows; unused by the mixed and split-BF16 forms).
 static void plan_forward_on(Plan* p, const double* re, const double* im, double* cre, double* cim, int F, Fmt fmt,
@@ -372,7 +377,7 @@ static void plan_forward_on(Plan* p, const double* re, const double* im, double*
     if (p->precision == S2AMD_MIXED || p->precision == S2AMD_SPLIT_BF16)
         forward_mixed(p->c, p->g, re, im, cre, cim, F, fmt, X, s, tm);
     else if (use_fast(p, F))
-        forward_fast(p->c, p->g, re, im, cre, cim, F, fmt, X, Cb, s, tm);
+        forward_fast(p->c, gemm_of(p, F), re, im, cre, cim, F, fmt, X, Cb, s, tm);
     else
         forward_fp64(p->c, p->t, re, im, cre, cim, F, fmt, (double2*)X, (double2*)Cb, s, tm);
 }
@@ -427,7 +432,7 @@ static void plan_inverse(Plan* p, const double* cre, const double* cim, double* 
     if (p->precision == S2AMD_MIXED || p->precision == S2AMD_SPLIT_BF16)
         inverse_mixed(p->c, p->g, cre, cim, re, im, F, fmt, p->X.p, s, &p->timer);
     else if (use_fast(p, F))
-        inverse_fast(p->c, p->g, cre, cim, re, im, F, fmt, p->X.p, p->Cb.p, s, &p->timer);
+        inverse_fast(p->c, gemm_of(p, F), cre, cim, re, im, F, fmt, p->X.p, p->Cb.p, s, &p->timer);
     else
         inverse_fp64(p->c, p->t, cre, cim, re, im, F, fmt, p->X.as<double2>(), p->Cb.as<double2>(), s, &p->timer);
 }
@@ -1072,7 +1077,16 @@ extern "C" int s2amd_plan_create(s2amd_plan** out, int bw, int cutoff, int max_f
                 split_tables_create(p->g, p->c, s);
             } else {
                 p->fast = fast_supported(bw, cutoff, precision);
-                if (p->fast) gemm_tables_create(p->g, p->t, precision, s);
+                // one field at bw >= 512 runs on the per-field kernels (use_fast)
+                const bool one = precision == S2AMD_FP64 && max_fields == 1 && bw >= 512;
+                if (p->fast && !one) {
+                    const int least = n64_min_fields(bw);
+                    if (n64_supported(bw, precision) && max_fields >= least) {
+                        p->dense_min = least;
+                        n64_tables_create(p->gd, p->t, p->c, s);
+                    }
+                    if (p->dense_min != 1) gemm_tables_create(p->g, p->t, precision, s);
+                }
             }
             const size_t N = 2 * (size_t)bw, F = max_fields;
             // large enough for the fast layouts and for the FP64 zonal transform
@@ -1088,6 +1102,7 @@ extern "C" int s2amd_plan_create(s2amd_plan** out, int bw, int cutoff, int max_f
             consts_destroy(p->c);
             tables_destroy(p->t);
             gemm_tables_destroy(p->g);
+            gemm_tables_destroy(p->gd);
             for (DBuf* b : {&p->X, &p->Cb, &p->cr, &p->ci, &p->zr, &p->zi}) b->release();
             throw;
         }
@@ -1128,6 +1143,7 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
         const bool mixed = p->precision == S2AMD_MIXED;
         if (!gemm && !mixed) return;  // nothing to choose for this plan and field count
         const size_t N = 2 * (size_t)p->bw, F = nfields;
+        GemmTables& g = gemm_of(p, nfields);
         struct Scratch {  // temporary fields, freed on every exit
             DBuf re, im, cr, ci;
             ~Scratch() {
@@ -1141,7 +1157,7 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
             ~Restore() {
                 if (!done) g.t_ncb = ncb, g.t_ct = ct, g.t_gj = gj;
             }
-        } keep{p->g, p->g.t_ncb, p->g.t_ct, p->g.t_gj};
+        } keep{g, g.t_ncb, g.t_ct, g.t_gj};
         t.re.reserve(sizeof(double) * N * N * F);
         t.im.reserve(sizeof(double) * N * N * F);
         t.cr.reserve(sizeof(double) * p->bw * p->bw * F);
@@ -1153,22 +1169,22 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
         float best = 1e30f;
         if (gemm) {
             int bn = 0, bc = 0;
-            for (const auto& tc : gemm_tile_choices(p->bw, p->precision)) {
-                p->g.t_ncb = tc.first;
-                p->g.t_ct = tc.second;
+            for (const auto& tc : gemm_tile_choices(g)) {
+                g.t_ncb = tc.first;
+                g.t_ct = tc.second;
                 const float ms = run();
                 if (ms < best) best = ms, bn = tc.first, bc = tc.second;
             }
-            p->g.t_ncb = bn;
-            p->g.t_ct = bc;
+            g.t_ncb = bn;
+            g.t_ct = bc;
         } else {
             int bg = 0;
             for (int gj : mix_gj_choices(p->bw)) {
-                p->g.t_gj = gj;
+                g.t_gj = gj;
                 const float ms = run();
                 if (ms < best) best = ms, bg = gj;
             }
-            p->g.t_gj = bg;
+            g.t_gj = bg;
         }
         S2_HIP(hipStreamSynchronize(s));
         keep.done = true;
@@ -1178,8 +1194,9 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
 extern "C" int s2amd_plan_tuning(const s2amd_plan* p, int* cols, int* col_tiles, int* ring_groups) {
     return run_plan("s2amd_plan_tuning", [&] {
         if (!p) throw ArgError{"plan is NULL"};
-        if (cols) *cols = p->g.t_ncb;
-        if (col_tiles) *col_tiles = p->g.t_ct;
+        const GemmTables& g = p->dense_min && p->gd.t_ncb ? p->gd : p->g;
+        if (cols) *cols = g.t_ncb;
+        if (col_tiles) *col_tiles = g.t_ct;
         if (ring_groups) *ring_groups = p->g.t_gj;
     });
 }
@@ -1193,6 +1210,7 @@ extern "C" int s2amd_plan_destroy(s2amd_plan* p) {
         consts_destroy(p->c);
         tables_destroy(p->t);
         gemm_tables_destroy(p->g);
+        gemm_tables_destroy(p->gd);
         for (DBuf* b : {&p->X, &p->Cb, &p->cr, &p->ci, &p->zr, &p->zi}) b->release();
         delete p;
     });
@@ -1203,7 +1221,7 @@ extern "C" size_t s2amd_plan_bytes(const s2amd_plan* p) {
     const size_t el = p->precision == S2AMD_FP64        ? sizeof(double)
                       : p->precision == S2AMD_SPLIT_BF16 ? sizeof(uint16_t)
                                                          : sizeof(float);  // GEMM table elements
-    return 2 * sizeof(double) * p->t.total + el * (p->g.nf + p->g.ni) + p->X.n + p->Cb.n + p->cr.n + p->ci.n +
+    return 2 * sizeof(double) * p->t.total + el * (p->g.nf + p->g.ni) + sizeof(double) * (p->gd.nf + p->gd.ni) + p->X.n + p->Cb.n + p->cr.n + p->ci.n +
            p->zr.n + p->zi.n;
 }
 

@@ -1,5 +1,7 @@
 // Batched GEMM path, FP64 or FP32 arithmetic (FP64 inputs and outputs either
-// way).  Power-of-two grids (N = 2*bw = 64 .. 2048):
+// way).  FP64 calls at bw <= 512 (from four fields above bw = 320) run the
+// dense GEMMs of s2_naive64.hip instead of the DCT and GEMM stages below,
+// around the same ring FFTs.  Power-of-two grids (N = 2*bw = 64 .. 2048):
 //
 //   k_fphi_fwd -> k_fdct_fwd -> k_gemm_fwd     forward  (ring FFT, DCT: s2_blocks.h)
 //   k_gemm_inv -> k_fdct_inv -> k_fphi_inv     inverse
@@ -544,7 +546,8 @@ __global__ __launch_bounds__(kThreads) void k_gemm_inv(const double* __restrict_
 // MFMAs and a block reads its order's table once per 64 columns.  The table
 // values of the next chunk are loaded before the current chunk's MFMAs.  Each
 // accumulator takes its K steps in the same ascending order as the kernels
-// above: the results are the same.
+// above: the results are the same.  FP32 plans only (FP64 ones take the dense
+// GEMMs at these sizes).
 constexpr int kKcCols = 64, kKc = 16, kKcNS = 1, kKcRS = kKc + 2;
 constexpr int kKcSteps = kKc / 4;                   // K steps of 4 per chunk
 
@@ -926,7 +929,9 @@ static void inv_launch(const DevConsts& c, const GemmTables& g, const double* cr
                (const GemmMeta*)g.meta, (R*)Cb, (T*)X, B, g.cut, mlo, F, ncb, (int)fmt);
 }
 
-std::vector<std::pair<int, int>> gemm_tile_choices(int bw, int prec) {
+std::vector<std::pair<int, int>> gemm_tile_choices(const GemmTables& g) {
+    if (g.n64) return {{16, 1}, {32, 2}};  // column tiles per wave
+    const int bw = g.bw, prec = g.prec;
     const int row = gemm_row(bw, prec), n0 = gemm_ncb(bw, prec);
     std::vector<std::pair<int, int>> v{{n0, gemm_ct(n0, bw)}};
     for (int n = 16; n <= 64; n <<= 1) {
@@ -943,13 +948,13 @@ static void gemm_tiles(const DevConsts& c, const GemmTables& g, int& ncb, bool& 
     two = (g.t_ncb ? g.t_ct : gemm_ct(ncb, c.bw)) == 2;
 }
 
-// The K-chunked kernels take the seminaive orders (m < cutoff) of calls of
+// The K-chunked kernels take the seminaive orders (m < cutoff) of FP32 calls of
 // many fields, bw in [128, 512] (at most sixteen 16-wide tiles per parity:
 // one per wave; at bw = 64 they were slower, 31.5 -> 34.0 us forward at 256
 // fields); the naive orders of a plan with cutoff < bw follow in a second
 // launch of the whole-row kernels.
 static bool kc_ok(const DevConsts& c, const GemmTables& g, int F) {
-    return g.cut > 0 && c.bw >= 128 && c.bw <= 512 && F >= 64;
+    return g.prec == 1 && g.cut > 0 && c.bw >= 128 && c.bw <= 512 && F >= 64;
 }
 // threads of a K-chunked block: one wave per 16-wide tile of a parity
 static int kc_threads(int B) { return B <= 256 ? 512 : 1024; }
@@ -958,15 +963,10 @@ static dim3 kc_grid(int B, int F) { return dim3((4 * F + kKcCols - 1) / kKcCols,
 
 void gemm_fwd_launch(const DevConsts& c, const GemmTables& g, const void* Cb, const void* X, double* cre, double* cim,
                      int F, Fmt fmt, hipStream_t s) {
+    if (g.n64) return n64_fwd_launch(c, g, (const double2*)X, cre, cim, F, fmt, s);
     if (kc_ok(c, g, F)) {
-        if (g.prec != 0)
-            (kc_threads(c.bw) == 512 ? k_gemm_fwd_kc<float, 512> : k_gemm_fwd_kc<float, 1024>)<<<kc_grid(c.bw, F), kc_threads(c.bw), 0, s>>>((const float*)Cb, (const float*)g.af,
-                                                                     (const GemmMeta*)g.meta, cre, cim, c.bw, g.cut, F,
-                                                                     (int)fmt);
-        else
-            (kc_threads(c.bw) == 512 ? k_gemm_fwd_kc<double, 512> : k_gemm_fwd_kc<double, 1024>)<<<kc_grid(c.bw, F), kc_threads(c.bw), 0, s>>>((const double*)Cb, (const double*)g.af,
-                                                                      (const GemmMeta*)g.meta, cre, cim, c.bw, g.cut, F,
-                                                                      (int)fmt);
+        (kc_threads(c.bw) == 512 ? k_gemm_fwd_kc<float, 512> : k_gemm_fwd_kc<float, 1024>)<<<kc_grid(c.bw, F), kc_threads(c.bw), 0, s>>>(
+            (const float*)Cb, (const float*)g.af, (const GemmMeta*)g.meta, cre, cim, c.bw, g.cut, F, (int)fmt);
         S2_HIP(hipGetLastError());
         if (g.cut == c.bw) return;
     }
@@ -984,15 +984,10 @@ void gemm_fwd_launch(const DevConsts& c, const GemmTables& g, const void* Cb, co
 
 void gemm_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, void* Cb, void* X,
                      int F, Fmt fmt, hipStream_t s) {
+    if (g.n64) return n64_inv_launch(c, g, cre, cim, (double2*)X, F, fmt, s);
     if (kc_ok(c, g, F)) {
-        if (g.prec != 0)
-            (kc_threads(c.bw) == 512 ? k_gemm_inv_kc<float, 512> : k_gemm_inv_kc<float, 1024>)<<<kc_grid(c.bw, F), kc_threads(c.bw), 0, s>>>(cre, cim, (const float*)g.ai,
-                                                                     (const GemmMeta*)g.meta, (float*)Cb, c.bw, g.cut, F,
-                                                                     (int)fmt);
-        else
-            (kc_threads(c.bw) == 512 ? k_gemm_inv_kc<double, 512> : k_gemm_inv_kc<double, 1024>)<<<kc_grid(c.bw, F), kc_threads(c.bw), 0, s>>>(cre, cim, (const double*)g.ai,
-                                                                      (const GemmMeta*)g.meta, (double*)Cb, c.bw, g.cut, F,
-                                                                      (int)fmt);
+        (kc_threads(c.bw) == 512 ? k_gemm_inv_kc<float, 512> : k_gemm_inv_kc<float, 1024>)<<<kc_grid(c.bw, F), kc_threads(c.bw), 0, s>>>(
+            cre, cim, (const float*)g.ai, (const GemmMeta*)g.meta, (float*)Cb, c.bw, g.cut, F, (int)fmt);
         S2_HIP(hipGetLastError());
         if (g.cut == c.bw) return;
     }

@@ -102,17 +102,18 @@ struct DevConsts {
 // path (s2_fast.hip) and the mixed form (s2_mixed.hip).  Entry m*2+p describes order m, degrees l = m+p+2i.
 struct GemmMeta {
     int Lp;     // number of degrees in the class
-    int Kf;     // seminaive: cosine terms of its last (longest) row
+    int Kf;     // seminaive: cosine terms of its last (longest) row; dense FP64: tiles per parity of its order pair
     long offF;  // seminaive: AF(m,p) [roundup4(Kf)][roundup16(Lp)]; mixed: NF(m), both parities
     long offI;  // seminaive: AI(m,p) [roundup4(Lp)][roundup16(bw/2)]; mixed: NI(m,p)
-    int n0;     // mixed: 16-degree tiles per parity, ceil(Lp(m,0)/16)
-    int ki;     // mixed: rows of NI(m,p), Lp padded to whole 16-degree chunks
+    int n0;     // mixed, dense FP64: 16-degree tiles per parity, ceil(Lp(m,0)/16)
+    int ki;     // mixed: rows of NI(m,p), Lp padded to whole 16-degree chunks; dense FP64: K steps of NI(m)
 };
 
 struct GemmTables {
     int bw = 0, prec = 0;  // prec 0: FP64, 1: FP32 (seminaive); 2: FP32 naive (mixed form); 3: split BF16 naive
     int cut = 0;           // prec 0, 1: orders m >= cut are naive (sampled P_l^m tables)
     bool gen = false;      // prec 0, bw not a power of two: natural-order Cb rows of the per-field path
+    bool n64 = false;      // prec 0: dense FP64 tables for every order (s2_naive64.hip; cut = 0)
     // tile choices from s2amd_plan_autotune (0: the built-in heuristic)
     int t_ncb = 0, t_ct = 0;  // prec 0, 1: data columns per GEMM block, column tiles per table load
     int t_gj = 0;             // prec 2: 64-ring groups per inverse GEMM block
@@ -223,11 +224,19 @@ void gemm_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre,
                      int F, Fmt fmt, hipStream_t s);
 // Tile shapes the GEMMs accept at bw: (columns per block, column tiles per
 // table load), the heuristic's choice first.
-std::vector<std::pair<int, int>> gemm_tile_choices(int bw, int prec);
+std::vector<std::pair<int, int>> gemm_tile_choices(const GemmTables& g);
 // 64-ring groups per mixed inverse GEMM block that bw admits, the default first.
 std::vector<int> mix_gj_choices(int bw);
 void gemm_tables_create(GemmTables& g, const DevTables& t, int prec, hipStream_t s);
 void gemm_tables_destroy(GemmTables& g);
+// ---- dense FP64 Legendre GEMMs (s2_naive64.hip) ---------------------------
+bool n64_supported(int bw, int prec);  // FP64, bw in [16, 512]
+int n64_min_fields(int bw);            // fields per call from which they beat the seminaive tables
+void n64_tables_create(GemmTables& g, const DevTables& t, const DevConsts& c, hipStream_t s);
+void n64_fwd_launch(const DevConsts& c, const GemmTables& g, const double2* X, double* cre, double* cim, int F, Fmt fmt,
+                    hipStream_t s);
+void n64_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, double2* X, int F,
+                    Fmt fmt, hipStream_t s);
 size_t fast_x_bytes(int bw, int prec);   // scratch X per field
 size_t fast_cb_bytes(int bw, int prec);  // scratch Cb per field
 void forward_fast(const DevConsts& c, const GemmTables& g, const double* re, const double* im, double* cre,

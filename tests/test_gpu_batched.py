@@ -534,3 +534,46 @@ def test_real_inverse_does_not_depend_on_earlier_calls(env, bw, F, prec):
     later = real_inverse(plan)
     plan.close()
     assert torch.equal(fresh[0], later[0]) and torch.equal(fresh[1], later[1])
+
+
+@pytest.mark.parametrize("bw,F,cutoff,fmt", [
+    (16, 1, 16, 0), (17, 3, 17, 1), (31, 9, 31, 0), (33, 70, 33, 0), (48, 17, 0, 1), (64, 129, 64, 0),
+    (127, 19, 127, 0), (128, 18, 128, 1), (128, 19, 128, 0), (129, 20, 40, 0), (129, 65, 129, 1), (160, 64, 160, 0),
+    (255, 7, 255, 1), (257, 8, 257, 0), (288, 16, 288, 1), (289, 17, 100, 0), (320, 2, 320, 0), (321, 3, 321, 0),
+    (321, 4, 321, 1), (511, 5, 511, 0)])
+def test_dense_fp64_legendre(env, O, bw, F, cutoff, fmt):
+    # The dense FP64 GEMMs at the edges of their tiles, of their instances
+    # (direct, K-chunked with 32 and with 64 columns per block, one or two
+    # halves, a middle order, a partial last column block) and of the rule
+    # that picks the table set above bw = 320: the first and last fields
+    # against the oracle, and up to bw = 320 bit for bit against calls of one
+    # field, whose sums take the same order.
+    S, torch, dev = env
+    n, kind = 2 * bw, 2 if fmt == 1 else 0
+    ends = sorted({0, F - 1})
+    coeffs = {f: O.make_coeffs(500 + f, bw, kind) for f in ends}
+    print(f"dense fp64 bw={bw} F={F} cutoff={cutoff} fmt={fmt}", flush=True)
+    cre = to_dev(torch, dev, [coeffs.get(f, coeffs[0])[0] for f in range(F)])
+    cim = to_dev(torch, dev, [coeffs.get(f, coeffs[0])[1] for f in range(F)])
+    gre = torch.empty((F, n, n), dtype=torch.float64, device=dev)
+    gim = torch.empty_like(gre)
+    c2r, c2i = torch.empty_like(cre), torch.empty_like(cim)
+    plan = S.Plan(bw, F, precision=0, cutoff=cutoff)
+    plan.inverse(cre, cim, gre, gim, data_format=fmt)
+    plan.forward(gre, gim, c2r, c2i, data_format=fmt)
+    torch.cuda.synchronize()
+    plan.close()
+    one = S.Plan(bw, 1, precision=0, cutoff=cutoff)
+    for f in ends:
+        og = O.inv_fst(coeffs[f][0], coeffs[f][1], bw, data_format=fmt, cutoff=cutoff)
+        assert crel(gre[f].cpu().numpy().ravel(), gim[f].cpu().numpy().ravel(), *og) < 1e-11
+        oc = O.fst(gre[f].cpu().numpy().ravel(), gim[f].cpu().numpy().ravel(), bw, data_format=fmt, cutoff=cutoff)
+        assert crel(c2r[f].cpu().numpy(), c2i[f].cpu().numpy(), *oc) < 1e-11
+        if bw <= 320:
+            a, b = torch.empty_like(gre[f:f + 1]), torch.empty_like(gim[f:f + 1])
+            one.inverse(cre[f:f + 1], cim[f:f + 1], a, b, data_format=fmt)
+            assert torch.equal(a, gre[f:f + 1]) and torch.equal(b, gim[f:f + 1])
+            a, b = torch.empty_like(cre[f:f + 1]), torch.empty_like(cim[f:f + 1])
+            one.forward(gre[f:f + 1], gim[f:f + 1], a, b, data_format=fmt)
+            assert torch.equal(a, c2r[f:f + 1]) and torch.equal(b, c2i[f:f + 1])
+    one.close()
