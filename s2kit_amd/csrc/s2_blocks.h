@@ -15,6 +15,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "s2_complex.h"
 #include "s2_internal.h"
 
@@ -231,10 +233,16 @@ __device__ __forceinline__ T* stage_twiddles(unsigned char* smem, const T* __res
 // FFT-type kernels.  grid.y = field, block = NTH (default kThreads) threads,
 // LDS = N twiddles + rows*(N+1) values
 // ---------------------------------------------------------------------------
+// REAL data (real != 0): order rows m < bw only, in both ring FFTs.  The
+// forward stores no other row (the Legendre stages of REAL data read none),
+// and the inverse takes row N-m as the conjugate of row m: half of X is
+// neither written nor read (measured REAL, us forward / inverse ring FFT and
+// inverse GEMM: mixed bw=128 x512 146 / 177, 89 -> 119 / 147, 64; bw=256 x256
+// 279 / 320, 176 -> 227 / 268, 133; FP64 bw=128 x64 step 118 -> 103).
 template <typename R, int V, int NTH = kThreads, bool NTF = false>
 __global__ __launch_bounds__(NTH) void k_fphi_fwd(const double* __restrict__ re, const double* __restrict__ im,
                                                        typename Cplx<R>::type* __restrict__ X, int lgN,
-                                                       const typename Cplx<R>::type* __restrict__ tw) {
+                                                       const typename Cplx<R>::type* __restrict__ tw, int real) {
     using T = typename Cplx<R>::type;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int E = V * NTH;
@@ -262,19 +270,22 @@ __global__ __launch_bounds__(NTH) void k_fphi_fwd(const double* __restrict__ re,
     }
     __syncthreads();
     fft_block<T, -1, V, NTH>(a, lgN, S, twl);
-    {
-        T v[V];
+    auto store = [&](auto cnt) __attribute__((always_inline)) {  // the first cnt/V of the rows
+        constexpr int U = decltype(cnt)::value;
+        T v[U];
 #pragma unroll
-        for (int u = 0; u < V; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int idx = threadIdx.x + u * NTH;
             v[u] = a[(idx & (rpb - 1)) * S + (idx >> lgrpb)];
         }
 #pragma unroll
-        for (int u = 0; u < V; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int idx = threadIdx.x + u * NTH;
             st_stream_c<NTF>(X + ((size_t)f * N + (idx >> lgrpb)) * N + j0 + (idx & (rpb - 1)), v[u]);
         }
-    }
+    };
+    if (real) store(std::integral_constant<int, V / 2>{});
+    else store(std::integral_constant<int, V>{});
 }
 
 // Weighted DCT-II of each order row (the data of DLTSemi, seminaive.c:161-176),
@@ -343,10 +354,10 @@ __global__ __launch_bounds__(NTH) void k_fdct_fwd(const typename Cplx<R>::type* 
 // DCT-III of each order row, x sin(theta) for odd orders, row signs and
 // 1/sqrt(2pi) (InvDLTSemi's tail, seminaive.c:107-114, and
 // FST_semi_memo.c:301-348): V[k] = e^{+i pi k/2N} (X[k] - i X[N-k]), one
-// N-point inverse FFT, even/odd unshuffle.  REAL data also fills row N-r.
+// N-point inverse FFT, even/odd unshuffle.
 template <typename R, int V, int NTH = kThreads>
 __global__ __launch_bounds__(NTH) void k_fdct_inv(const R* __restrict__ Cb, typename Cplx<R>::type* __restrict__ X,
-                                                  const R* __restrict__ sinv, int lgN, int cut, int nrows, int fmt,
+                                                  const R* __restrict__ sinv, int lgN, int cut, int nrows,
                                                   const typename Cplx<R>::type* __restrict__ tw,
                                                   const typename Cplx<R>::type* __restrict__ ph) {
     using T = typename Cplx<R>::type;
@@ -442,9 +453,7 @@ __global__ __launch_bounds__(NTH) void k_fdct_inv(const R* __restrict__ Cb, type
         R sc = inv_s2pi;
         if (am & 1) sc *= sv[u];
         if (r > B && (r & 1)) sc = -sc;
-        const T y = cscale(yv, sc);
-        X[((size_t)f * N + r) * N + j] = y;
-        if (fmt == 1 && r > 0) X[((size_t)f * N + (N - r)) * N + j] = cconj(y);
+        X[((size_t)f * N + r) * N + j] = cscale(yv, sc);
     }
 }
 
@@ -453,7 +462,7 @@ __global__ __launch_bounds__(NTH) void k_fdct_inv(const R* __restrict__ Cb, type
 template <typename R, int V, int NTH = kThreads, bool W16 = false>
 __global__ __launch_bounds__(NTH) void k_fphi_inv(const typename Cplx<R>::type* __restrict__ X,
                                                        double* __restrict__ re, double* __restrict__ im, int lgN,
-                                                       const typename Cplx<R>::type* __restrict__ tw) {
+                                                       const typename Cplx<R>::type* __restrict__ tw, int real) {
     using T = typename Cplx<R>::type;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int E = V * NTH;
@@ -469,7 +478,22 @@ __global__ __launch_bounds__(NTH) void k_fphi_inv(const typename Cplx<R>::type* 
     // 0.35 -> 0.39 ms)
     constexpr bool kLate = sizeof(R) == 8 || W16;
     if constexpr (!kLate) stage_twiddles<T, NTH>(smem, tw, N);
-    {
+    if (real) {  // rows r < B, and their conjugates at N - r
+        T v[V / 2];
+#pragma unroll
+        for (int u = 0; u < V / 2; ++u) {
+            const int idx = threadIdx.x + u * NTH;
+            v[u] = X[((size_t)f * N + (idx >> lgrpb)) * N + j0 + (idx & (rpb - 1))];
+        }
+        if constexpr (kLate) stage_twiddles<T, NTH>(smem, tw, N);
+#pragma unroll
+        for (int u = 0; u < V / 2; ++u) {
+            const int idx = threadIdx.x + u * NTH, r = idx >> lgrpb;
+            T* row = a + (idx & (rpb - 1)) * S;
+            row[r] = v[u];
+            row[r ? N - r : B] = r ? cconj(v[u]) : mk<T>(0, 0);
+        }
+    } else {
         T v[V];
 #pragma unroll
         for (int u = 0; u < V; ++u) {

@@ -465,7 +465,7 @@ __device__ __forceinline__ void gemm_inv_semi(R* __restrict__ Cd, const double* 
 // X: per ring j < bw the parity sums E (p = 0) and O (p = 1) over the table
 // rows (which carry 1/sqrt(2pi)) give ring j <- E+O and ring N-1-j <- E-O.
 // Row N-m of an odd order carries a minus sign (FST_semi_memo.c:301-348),
-// put on its coefficients; REAL data also fills the conjugate row N-m.
+// put on its coefficients.
 template <typename R, int CT>
 __device__ __forceinline__ void gemm_inv_naive(R* __restrict__ Cd, const double* __restrict__ cre,
                                                const double* __restrict__ cim, const R* __restrict__ AI,
@@ -482,7 +482,6 @@ __device__ __forceinline__ void gemm_inv_naive(R* __restrict__ Cd, const double*
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nctg = (ncb >> 4) / CT;
     const int ntt = B16 >> 4;
-    const bool mirror = fmt == 1 && m > 0;
     for (int item = item0(wave); item < ntt * nctg; item += item_step()) {
         const int tt = item / nctg, ct = item - tt * nctg;
         const int t0 = tt * 16, c0 = ct * 16 * CT;
@@ -505,11 +504,6 @@ __device__ __forceinline__ void gemm_inv_naive(R* __restrict__ Cd, const double*
                 const R lo = e[c][r] + o[c][r], hi = e[c][r] - o[c][r];
                 xr[2 * j] = lo;
                 xr[2 * (N - 1 - j)] = hi;
-                if (mirror) {  // conj into row N-m
-                    R* xm = reinterpret_cast<R*>(X + ((size_t)f * N + (N - m)) * N) + comp;
-                    xm[2 * j] = comp ? -lo : lo;
-                    xm[2 * (N - 1 - j)] = comp ? -hi : hi;
-                }
             }
     }
 }
@@ -1016,25 +1010,25 @@ static void fwd_impl(const DevConsts& c, const GemmTables& g, const double* re, 
     const T* tw = (const T*)(sizeof(R) == 8 ? (const void*)c.tw : (const void*)c.tw32);
     const T* ph = (const T*)(sizeof(R) == 8 ? (const void*)c.ph : (const void*)c.ph32);
     const R* ws = (const R*)(sizeof(R) == 8 ? (const void*)c.w_semi : (const void*)c.w_semi32);
-    const int few = few_field_threads<V>(N, F);
+    const int few = few_field_threads<V>(N, F), real = fmt == Fmt::Real;
     const int rpf = few ? V * few / N : 0;  // rings per one-wave block
     const size_t ldf = few ? sizeof(T) * ((size_t)rpf * (N + 1) + N) : 0;
     {
         Span sp(tm, ST_PHI_FWD, s);
         // 512-thread blocks (twice the rings, full 128-byte row segments) when a block still holds whole rows
         if (few == 64) {
-            launch_lds(k_fphi_fwd<R, V, 64>, dim3(N / rpf, F), 64, ldf, s, re, im, X, lgN, tw);
+            launch_lds(k_fphi_fwd<R, V, 64>, dim3(N / rpf, F), 64, ldf, s, re, im, X, lgN, tw, real);
         } else if (few == 128) {
-            launch_lds(k_fphi_fwd<R, V, 128>, dim3(N / rpf, F), 128, ldf, s, re, im, X, lgN, tw);
+            launch_lds(k_fphi_fwd<R, V, 128>, dim3(N / rpf, F), 128, ldf, s, re, im, X, lgN, tw, real);
         } else if ((long)N * N >= 512L * V) {
             const int rp2 = V * 512 / N;
             const size_t l2 = sizeof(T) * ((size_t)rp2 * (N + 1) + N);
             if (k_fphi_fwd_nt(rp2, sizeof(T)))
-                launch_lds(k_fphi_fwd<R, V, 512, true>, dim3(N / rp2, F), 512, l2, s, re, im, X, lgN, tw);
+                launch_lds(k_fphi_fwd<R, V, 512, true>, dim3(N / rp2, F), 512, l2, s, re, im, X, lgN, tw, real);
             else
-                launch_lds(k_fphi_fwd<R, V, 512>, dim3(N / rp2, F), 512, l2, s, re, im, X, lgN, tw);
+                launch_lds(k_fphi_fwd<R, V, 512>, dim3(N / rp2, F), 512, l2, s, re, im, X, lgN, tw, real);
         } else {
-            launch_lds(k_fphi_fwd<R, V>, dim3(N / rpb, F), kThreads, lds, s, re, im, X, lgN, tw);
+            launch_lds(k_fphi_fwd<R, V>, dim3(N / rpb, F), kThreads, lds, s, re, im, X, lgN, tw, real);
         }
     }
     // weighted DCT of the seminaive order rows only
@@ -1075,7 +1069,7 @@ static void inv_impl(const DevConsts& c, const GemmTables& g, const double* cre,
     const T* tw = (const T*)(sizeof(R) == 8 ? (const void*)c.tw : (const void*)c.tw32);
     const T* ph = (const T*)(sizeof(R) == 8 ? (const void*)c.ph : (const void*)c.ph32);
     const R* sv = (const R*)(sizeof(R) == 8 ? (const void*)c.sinv : (const void*)c.sinv32);
-    const int few = few_field_threads<V>(N, F);
+    const int few = few_field_threads<V>(N, F), real = fmt == Fmt::Real;
     const int rpf = few ? V * few / N : 0;  // rings per one-wave block
     const size_t ldf = few ? sizeof(T) * ((size_t)rpf * (N + 1) + N) : 0;
     {
@@ -1088,32 +1082,31 @@ static void inv_impl(const DevConsts& c, const GemmTables& g, const double* cre,
         Span sp(tm, ST_DCT_INV, s);
         if (few == 64) {
             launch_lds(k_fdct_inv<R, V, 64>, dim3((nrows + rpf - 1) / rpf, F), 64, ldf, s, (const R*)Cb, X, sv, lgN,
-                       cut, nrows, (int)fmt, tw, ph);
+                       cut, nrows, tw, ph);
         } else if (few == 128) {
             launch_lds(k_fdct_inv<R, V, 128>, dim3((nrows + rpf - 1) / rpf, F), 128, ldf, s, (const R*)Cb, X, sv, lgN,
-                       cut, nrows, (int)fmt, tw, ph);
+                       cut, nrows, tw, ph);
         } else if ((long)N * N >= 512L * V) {
             const int rp2 = V * 512 / N;
             launch_lds(k_fdct_inv<R, V, 512>, dim3((nrows + rp2 - 1) / rp2, F), 512,
-                       sizeof(T) * ((size_t)rp2 * (N + 1) + N), s, (const R*)Cb, X, sv, lgN, cut, nrows, (int)fmt, tw,
-                       ph);
+                       sizeof(T) * ((size_t)rp2 * (N + 1) + N), s, (const R*)Cb, X, sv, lgN, cut, nrows, tw, ph);
         } else {
             launch_lds(k_fdct_inv<R, V>, dim3((nrows + rpb - 1) / rpb, F), kThreads, lds, s, (const R*)Cb, X, sv, lgN,
-                       cut, nrows, (int)fmt, tw, ph);
+                       cut, nrows, tw, ph);
         }
     }
     {
         Span sp(tm, ST_PHI_INV, s);
         if (few == 64) {
-            launch_lds(k_fphi_inv<R, V, 64>, dim3(N / rpf, F), 64, ldf, s, (const T*)X, re, im, lgN, tw);
+            launch_lds(k_fphi_inv<R, V, 64>, dim3(N / rpf, F), 64, ldf, s, (const T*)X, re, im, lgN, tw, real);
         } else if (few == 128) {
-            launch_lds(k_fphi_inv<R, V, 128>, dim3(N / rpf, F), 128, ldf, s, (const T*)X, re, im, lgN, tw);
+            launch_lds(k_fphi_inv<R, V, 128>, dim3(N / rpf, F), 128, ldf, s, (const T*)X, re, im, lgN, tw, real);
         } else if ((long)N * N >= 512L * V) {
             const int rp2 = V * 512 / N;
             launch_lds(k_fphi_inv<R, V, 512>, dim3(N / rp2, F), 512, sizeof(T) * ((size_t)rp2 * (N + 1) + N), s,
-                       (const T*)X, re, im, lgN, tw);
+                       (const T*)X, re, im, lgN, tw, real);
         } else {
-            launch_lds(k_fphi_inv<R, V>, dim3(N / rpb, F), kThreads, lds, s, (const T*)X, re, im, lgN, tw);
+            launch_lds(k_fphi_inv<R, V>, dim3(N / rpb, F), kThreads, lds, s, (const T*)X, re, im, lgN, tw, real);
         }
     }
 }

@@ -446,7 +446,7 @@ __device__ __forceinline__ int row_of(int q, int N, int cut) { return q < cut ? 
 template <typename T, int MODE>
 __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) void k_phi_fwd(const double* __restrict__ re, const double* __restrict__ im,
                                                  T* __restrict__ X, int N, int logN, int pow2, int rpb,
-                                                 const T* __restrict__ tw) {
+                                                 const T* __restrict__ tw, int real) {
     extern __shared__ __align__(16) unsigned char smem[];
     T* a = reinterpret_cast<T*>(smem);
     const int RS = row_stride<MODE>(N, logN);
@@ -481,7 +481,8 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     __syncthreads();
     T* r = fft_rows<T, -1, MODE>(a, b, N, logN, pow2, nr, twp, tw);
     const unsigned long long mnr = magic16(nr);
-    for (int i = threadIdx.x; i < tot; i += blockDim.x) {
+    const int out = real ? tot >> 1 : tot;  // REAL data: rows below bw (see k_fphi_fwd)
+    for (int i = threadIdx.x; i < out; i += blockDim.x) {
         const int row = div16(i, mnr), jl = i - row * nr;
         X[((size_t)f * N + row) * N + j0 + jl] = r[jl * RS + row];
     }
@@ -1059,12 +1060,12 @@ __global__ __launch_bounds__(256) void k_leg_inv(const double* __restrict__ cre,
 
 // DCT-III of every seminaive order row (inputs 0..B-1, zero above), then
 // x sin(theta) for odd orders, x (-1) on odd negative rows, x 1/sqrt(2pi).
-// REAL mirrors row N-m = conj(row m).  grid (ceil(nrows/rpb), F).
+// grid (ceil(nrows/rpb), F).
 template <typename T, int MODE>
 __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) void k_dct_inv(const T* __restrict__ Cb, T* __restrict__ X,
                                                  const T* __restrict__ tw, const T* __restrict__ ph,
                                                  const double* __restrict__ sinv, int N, int logN, int pow2, int B,
-                                                 int cut, int nrows, int rpb, int fmt, int planar) {
+                                                 int cut, int nrows, int rpb, int planar) {
     extern __shared__ __align__(16) unsigned char smem[];
     T* a = reinterpret_cast<T*>(smem);
     const int RS = row_stride<MODE>(N, logN);
@@ -1123,14 +1124,12 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
         R sc = inv_s2pi;
         if (am & 1) sc *= (R)sinv[j];
         if (r > B && (r & 1)) sc = -sc;
-        const T y = cscale(u[rl * RS + n], sc);
-        X[((size_t)f * N + r) * N + j] = y;
-        if (fmt == 1 && r > 0) X[((size_t)f * N + (N - r)) * N + j] = cconj(y);
+        X[((size_t)f * N + r) * N + j] = cscale(u[rl * RS + n], sc);
     }
 }
 
 // Dense synthesis of orders m >= cut (InvDLTNaive), with the same row
-// signs / scaling / REAL mirror as k_dct_inv.  grid (B-cut, ceil(F/fc)).
+// signs and scaling as k_dct_inv.  grid (B-cut, ceil(F/fc)).
 __global__ __launch_bounds__(256) void k_naive_inv(const double* __restrict__ cre, const double* __restrict__ cim,
                                                    const double* __restrict__ P, const long* __restrict__ toff,
                                                    double2* __restrict__ X, int N, int B, int cut, int F, int fc,
@@ -1162,19 +1161,17 @@ __global__ __launch_bounds__(256) void k_naive_inv(const double* __restrict__ cr
         const int r = s ? N - m : m;
         double sc = inv_s2pi;
         if (r > B && (r & 1)) sc = -sc;
-        const double2 y = make_double2(yr * sc, yi * sc);
-        const int f = f0 + fl;
-        X[((size_t)f * N + r) * N + j] = y;
-        if (fmt == 1 && r > 0) X[((size_t)f * N + (N - r)) * N + j] = make_double2(y.x, -y.y);
+        X[((size_t)(f0 + fl) * N + r) * N + j] = make_double2(yr * sc, yi * sc);
     }
 }
 
 // Inverse ring FFT (+i, unnormalised) per ring; row B (Nyquist) is zero.
+// REAL data: rows below bw only (see k_fphi_fwd), row N-m the conjugate of m.
 // grid (ceil(N/rpb), F).
 template <typename T, int MODE>
 __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) void k_phi_inv(const T* __restrict__ X, double* __restrict__ re,
                                                  double* __restrict__ im, int N, int logN, int pow2, int B, int rpb,
-                                                 const T* __restrict__ tw) {
+                                                 const T* __restrict__ tw, int real) {
     extern __shared__ __align__(16) unsigned char smem[];
     T* a = reinterpret_cast<T*>(smem);
     const int RS = row_stride<MODE>(N, logN);
@@ -1186,12 +1183,13 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     const int nr = min(rpb, N - j0);
     const int tot = nr * N;  // < 2^16 (div16)
     const unsigned long long mnr = magic16(nr);
-    for (int i0 = threadIdx.x; i0 < tot; i0 += FB * blockDim.x) {
+    const int in = real ? tot >> 1 : tot;
+    for (int i0 = threadIdx.x; i0 < in; i0 += FB * blockDim.x) {
         T v[FB];
 #pragma unroll
         for (int u = 0; u < FB; ++u) {
             const int i = i0 + u * blockDim.x;
-            if (i < tot) {
+            if (i < in) {
                 const int r = div16(i, mnr), jl = i - r * nr;
                 v[u] = (r == B) ? mk<T>(0, 0) : X[((size_t)f * N + r) * N + j0 + jl];
             }
@@ -1199,9 +1197,10 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
 #pragma unroll
         for (int u = 0; u < FB; ++u) {
             const int i = i0 + u * blockDim.x;
-            if (i < tot) {
+            if (i < in) {
                 const int r = div16(i, mnr), jl = i - r * nr;
                 a[jl * RS + r] = v[u];
+                if (real) a[jl * RS + (r ? N - r : B)] = r ? cconj(v[u]) : mk<T>(0, 0);
             }
         }
     }
@@ -1872,21 +1871,21 @@ static void reg_launch(const RegBlocks& rb, L&& launch) {
 // form's first and last stages at such bandwidths), on the register
 // mixed-radix or Bluestein instances; same order-major FP32 intermediate X
 // as the power-of-two register kernels.
-void ring_fft_fwd_f32(const DevConsts& c, const double* re, const double* im, float2* X, int F, hipStream_t s) {
+void ring_fft_fwd_f32(const DevConsts& c, const double* re, const double* im, float2* X, int F, Fmt fmt, hipStream_t s) {
     const int N = c.N;
     const FftCfg<float2> fg = fft_cfg<float2>(c);
     const int rpb = fg.rpb;
     fft_launch(fg, FFT_INSTANCES(k_phi_fwd, float2), dim3((N + rpb - 1) / rpb, F), s,
-               re, im, X, N, fg.lg, 0, rpb, fg.tw);
+               re, im, X, N, fg.lg, 0, rpb, fg.tw, (int)(fmt == Fmt::Real));
     S2_HIP(hipGetLastError());
 }
 
-void ring_fft_inv_f32(const DevConsts& c, const float2* X, double* re, double* im, int F, hipStream_t s) {
+void ring_fft_inv_f32(const DevConsts& c, const float2* X, double* re, double* im, int F, Fmt fmt, hipStream_t s) {
     const int N = c.N;
     const FftCfg<float2> fg = fft_cfg<float2>(c);
     const int rpb = fg.rpb;
     fft_launch(fg, FFT_INSTANCES(k_phi_inv, float2), dim3((N + rpb - 1) / rpb, F), s,
-               X, re, im, N, fg.lg, 0, c.bw, rpb, fg.tw);
+               X, re, im, N, fg.lg, 0, c.bw, rpb, fg.tw, (int)(fmt == Fmt::Real));
     S2_HIP(hipGetLastError());
 }
 
@@ -1902,11 +1901,11 @@ void forward_fp64(const DevConsts& c, const DevTables& t, const double* re, cons
     if (reg_rings(c))
         reg_launch(rb, [&](auto nth) {
             launch_lds(k_fphi_fwd<double, 8, decltype(nth)::value>, dim3(N / rb.rpb, F), rb.threads, rb.lds, s, re, im,
-                       X, c.logN, c.tw);
+                       X, c.logN, c.tw, f);
         });
     else
         fft_launch(fg, FFT_INSTANCES(k_phi_fwd, double2), dim3((N + rpb - 1) / rpb, F),
-                   s, re, im, X, N, fg.lg, c.pow2, rpb, fg.tw);
+                   s, re, im, X, N, fg.lg, c.pow2, rpb, fg.tw, (int)(fmt == Fmt::Real));
     S2_HIP(hipGetLastError());
     }
     if (cut > 0) {
@@ -1992,11 +1991,11 @@ void inverse_fp64(const DevConsts& c, const DevTables& t, const double* cre, con
         if (planar)
             reg_launch(rb, [&](auto nth) {
                 launch_lds(k_fdct_inv<double, 8, decltype(nth)::value>, dim3((nrows + rb.rpb - 1) / rb.rpb, F),
-                           rb.threads, rb.lds, s, (const double*)Cb, X, c.sinv, c.logN, cut, nrows, f, c.tw, c.ph);
+                           rb.threads, rb.lds, s, (const double*)Cb, X, c.sinv, c.logN, cut, nrows, c.tw, c.ph);
             });
         else
             fft_launch(fg, FFT_INSTANCES(k_dct_inv, double2),
-                       dim3((nrows + rpb - 1) / rpb, F), s, Cb, X, fg.tw, c.ph, c.sinv, N, fg.lg, c.pow2, B, cut, nrows, rpb, f, 0);
+                       dim3((nrows + rpb - 1) / rpb, F), s, Cb, X, fg.tw, c.ph, c.sinv, N, fg.lg, c.pow2, B, cut, nrows, rpb, 0);
         S2_HIP(hipGetLastError());
     }
     if (cut < B) {
@@ -2010,11 +2009,11 @@ void inverse_fp64(const DevConsts& c, const DevTables& t, const double* cre, con
     if (reg_rings(c))
         reg_launch(rb, [&](auto nth) {
             launch_lds(k_fphi_inv<double, 8, decltype(nth)::value>, dim3(N / rb.rpb, F), rb.threads, rb.lds, s,
-                       (const double2*)X, re, im, c.logN, c.tw);
+                       (const double2*)X, re, im, c.logN, c.tw, f);
         });
     else
         fft_launch(fg, FFT_INSTANCES(k_phi_inv, double2), dim3((N + rpb - 1) / rpb, F),
-                   s, X, re, im, N, fg.lg, c.pow2, B, rpb, fg.tw);
+                   s, X, re, im, N, fg.lg, c.pow2, B, rpb, fg.tw, (int)(fmt == Fmt::Real));
     S2_HIP(hipGetLastError());
 }
 
@@ -2027,7 +2026,7 @@ void forward_fp64_gemm(const DevConsts& c, const GemmTables& g, const double* re
     {
         Span sp(tm, ST_PHI_FWD, s);
         fft_launch(fg, FFT_INSTANCES(k_phi_fwd, double2), dim3((N + rpb - 1) / rpb, F),
-                   s, re, im, X, N, fg.lg, c.pow2, rpb, fg.tw);
+                   s, re, im, X, N, fg.lg, c.pow2, rpb, fg.tw, (int)(fmt == Fmt::Real));
         S2_HIP(hipGetLastError());
     }
     if (cut > 0) {
@@ -2044,7 +2043,7 @@ void forward_fp64_gemm(const DevConsts& c, const GemmTables& g, const double* re
 void inverse_fp64_gemm(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, double* re,
                        double* im, int F, Fmt fmt, double2* X, double2* Cb, hipStream_t s, StageTimer* tm) {
     check_launch_shape(c);
-    const int N = c.N, B = c.bw, cut = g.cut, f = (int)fmt;
+    const int N = c.N, B = c.bw, cut = g.cut;
     const FftCfg<double2> fg = fft_cfg<double2>(c);
     const int rpb = fg.rpb;
     {
@@ -2055,12 +2054,12 @@ void inverse_fp64_gemm(const DevConsts& c, const GemmTables& g, const double* cr
         const int nrows = (fmt == Fmt::Complex) ? 2 * cut - 1 : cut;
         Span sp(tm, ST_DCT_INV, s);
         fft_launch(fg, FFT_INSTANCES(k_dct_inv, double2),
-                       dim3((nrows + rpb - 1) / rpb, F), s, Cb, X, fg.tw, c.ph, c.sinv, N, fg.lg, c.pow2, B, cut, nrows, rpb, f, 1);
+                       dim3((nrows + rpb - 1) / rpb, F), s, Cb, X, fg.tw, c.ph, c.sinv, N, fg.lg, c.pow2, B, cut, nrows, rpb, 1);
         S2_HIP(hipGetLastError());
     }
     Span sp(tm, ST_PHI_INV, s);
     fft_launch(fg, FFT_INSTANCES(k_phi_inv, double2), dim3((N + rpb - 1) / rpb, F), s,
-               X, re, im, N, fg.lg, c.pow2, B, rpb, fg.tw);
+               X, re, im, N, fg.lg, c.pow2, B, rpb, fg.tw, (int)(fmt == Fmt::Real));
     S2_HIP(hipGetLastError());
 }
 

@@ -121,8 +121,7 @@ __device__ __forceinline__ void mix_fwd_store(const fvec4 (&acc)[2 * N0], double
 // (p = 1) at rings jbase + 16t + x16 of columns 4(lane/16) + r (the table
 // carries 1/sqrt(2pi), the operand the row sign); rows r, r+1 are the re, im
 // parts of one (field, sign) row.  Ring j <- E+O, ring N-1-j <- E-O (j < bw:
-// padded rings are not stored), and for REAL data the conjugate mirror row
-// N-m.
+// padded rings are not stored).
 template <int JT>
 __device__ __forceinline__ void mix_inv_store(const fvec4 (&acc)[2][JT], float2* __restrict__ X, int m, int cb,
                                               int jbase, int B, int F, int fmt) {
@@ -133,14 +132,12 @@ __device__ __forceinline__ void mix_inv_store(const fvec4 (&acc)[2][JT], float2*
     const int x16 = lane & 15, kq = lane >> 4;
     const int N = 2 * B;
     const int cpf = mix_cpf(m, fmt), ncols = F * cpf;
-    const bool mirror = fmt == 1 && m > 0;
 #pragma unroll
     for (int rr = 0; rr < 2; ++rr) {
         const int c = cb * kMixCols + wave * 16 + 4 * kq + 2 * rr;
         if (c >= ncols) continue;
         const int f = c / cpf, rem = c - f * cpf;
         float2* xr = X + ((size_t)f * N + ((rem >> 1) ? N - m : m)) * N;
-        float2* xm = X + ((size_t)f * N + (N - m)) * N;
         float2* plo = xr + jbase + x16;
         float2* phi = xr + (N - 1 - jbase - x16);
         const int r = 2 * rr;
@@ -150,17 +147,6 @@ __device__ __forceinline__ void mix_inv_store(const fvec4 (&acc)[2][JT], float2*
             const fvec4 e = acc[0][t], o = acc[1][t];
             plo[16 * t] = make_float2(e[r] + o[r], e[r + 1] + o[r + 1]);
             phi[-16 * t] = make_float2(e[r] - o[r], e[r + 1] - o[r + 1]);
-        }
-        if (mirror) {
-            float2* qlo = xm + jbase + x16;
-            float2* qhi = xm + (N - 1 - jbase - x16);
-#pragma unroll
-            for (int t = 0; t < JT; ++t) {
-                if (jbase + 16 * t + x16 >= B) continue;
-                const fvec4 e = acc[0][t], o = acc[1][t];
-                qlo[16 * t] = make_float2(e[r] + o[r], -(e[r + 1] + o[r + 1]));
-                qhi[-16 * t] = make_float2(e[r] - o[r], -(e[r + 1] - o[r + 1]));
-            }
         }
     }
 }

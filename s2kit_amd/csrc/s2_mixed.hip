@@ -515,24 +515,24 @@ void forward_mixed(const DevConsts& c, const GemmTables& g, const double* re, co
                    double* cim, int F, Fmt fmt, void* Xv, hipStream_t s, StageTimer* tm) {
     constexpr int V = 16;
     const int N = c.N, lgN = lg2(N);
-    const int rpb = V * kMixFftThreads / N;
+    const int rpb = V * kMixFftThreads / N, real = fmt == Fmt::Real;
     float2* X = (float2*)Xv;
     {
         Span sp(tm, ST_PHI_FWD, s);
         const size_t lds = sizeof(float2) * ((size_t)rpb * (N + 1) + N);
         if (!c.pow2) {  // mixed-radix FP32 ring FFTs
-            ring_fft_fwd_f32(c, re, im, X, F, s);
+            ring_fft_fwd_f32(c, re, im, X, F, fmt, s);
         } else if (rpb > N) {  // bw = 32: the 64 rings of a field in one 256-thread block
             constexpr int T2 = 256;
             const size_t l2 = sizeof(float2) * ((size_t)N * (N + 1) + N);
             launch_lds(k_fphi_fwd<float, V, T2, true>, dim3(1, F), T2, l2, s, re, im, X, lgN,
-                       (const float2*)c.tw32);
+                       (const float2*)c.tw32, real);
         } else if (k_fphi_fwd_nt(rpb, sizeof(float2)))
             launch_lds(k_fphi_fwd<float, V, kMixFftThreads, true>, dim3(N / rpb, F), kMixFftThreads, lds, s, re, im,
-                       X, lgN, (const float2*)c.tw32);
+                       X, lgN, (const float2*)c.tw32, real);
         else
             launch_lds(k_fphi_fwd<float, V, kMixFftThreads>, dim3(N / rpb, F), kMixFftThreads, lds, s, re, im, X,
-                       lgN, (const float2*)c.tw32);
+                       lgN, (const float2*)c.tw32, real);
     }
     {
         Span sp(tm, ST_LEG_FWD, s);
@@ -547,7 +547,7 @@ void inverse_mixed(const DevConsts& c, const GemmTables& g, const double* cre, c
                    double* im, int F, Fmt fmt, void* Xv, hipStream_t s, StageTimer* tm) {
     constexpr int V = 16;
     const int N = c.N, lgN = lg2(N);
-    const int rpb = V * kMixFftThreads / N;
+    const int rpb = V * kMixFftThreads / N, real = fmt == Fmt::Real;
     float2* X = (float2*)Xv;
     {
         Span sp(tm, ST_LEG_INV, s);
@@ -560,18 +560,18 @@ void inverse_mixed(const DevConsts& c, const GemmTables& g, const double* cre, c
         Span sp(tm, ST_PHI_INV, s);
         const size_t lds = sizeof(float2) * ((size_t)rpb * (N + 1) + N);
         if (!c.pow2) {  // mixed-radix FP32 ring FFTs
-            ring_fft_inv_f32(c, X, re, im, F, s);
+            ring_fft_inv_f32(c, X, re, im, F, fmt, s);
         } else if (rpb > N) {  // bw = 32: the 64 rings of a field in one 256-thread block
             constexpr int T2 = 256;
             const size_t l2 = sizeof(float2) * ((size_t)N * (N + 1) + N);
             launch_lds(k_fphi_inv<float, V, T2>, dim3(1, F), T2, l2, s, (const float2*)X, re, im, lgN,
-                       (const float2*)c.tw32);
+                       (const float2*)c.tw32, real);
         } else if ((((uintptr_t)re | (uintptr_t)im) & 15) == 0)
             launch_lds(k_fphi_inv<float, V, kMixFftThreads, true>, dim3(N / rpb, F), kMixFftThreads, lds, s,
-                       (const float2*)X, re, im, lgN, (const float2*)c.tw32);
+                       (const float2*)X, re, im, lgN, (const float2*)c.tw32, real);
         else
             launch_lds(k_fphi_inv<float, V, kMixFftThreads>, dim3(N / rpb, F), kMixFftThreads, lds, s,
-                       (const float2*)X, re, im, lgN, (const float2*)c.tw32);
+                       (const float2*)X, re, im, lgN, (const float2*)c.tw32, real);
     }
 }
 

@@ -92,12 +92,10 @@ __device__ __forceinline__ N64Out n64_out(int c, int m, int cpf, int B, int fmt,
 // re and im sums of column pair c (times sg), lane x16 the ring j of the first tile.
 template <int T>
 __device__ __forceinline__ void n64_inv_store(const dvec4 (&e)[T], const dvec4 (&o)[T], double2* __restrict__ X, int m,
-                                              int c, int r, double sg, int j, int B, int cpf, int fmt) {
+                                              int c, int r, double sg, int j, int B, int cpf) {
     const int N = 2 * B;
     const int f = c >> (cpf >> 1), rem = c & (cpf - 1);  // cpf is 2 or 4
     double2* xr = X + ((size_t)f * N + n64_row(rem, m, N)) * N;
-    double2* xm = X + ((size_t)f * N + (N - m)) * N;
-    const bool mirror = fmt == 1 && m > 0;  // REAL data: the conjugate row
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         const int jt = j + 16 * t;
@@ -106,10 +104,6 @@ __device__ __forceinline__ void n64_inv_store(const dvec4 (&e)[T], const dvec4 (
         const double2 hi = make_double2(sg * (e[t][r] - o[t][r]), sg * (e[t][r + 1] - o[t][r + 1]));
         xr[jt] = lo;
         xr[N - 1 - jt] = hi;
-        if (mirror) {
-            xm[jt] = make_double2(lo.x, -lo.y);
-            xm[N - 1 - jt] = make_double2(hi.x, -hi.y);
-        }
     }
 }
 // The inverse's operand row for accumulator row x16: lane (x16, kq) then holds
@@ -306,7 +300,7 @@ __device__ __forceinline__ void naive64_inv_direct(const double* __restrict__ cr
             const int col = (cg * CT + c) * 16 + 4 * kq + 2 * rr;
             const double sg = ((col & (cpf - 1)) >> 1) && (m & 1) ? -1.0 : 1.0;  // rows -m carry (-1)^m
             if (col < ncols)
-                n64_inv_store<RTW>(acc[c][0], acc[c][1], X, m, col, 2 * rr, sg, 16 * rt0 + x16, B, cpf, fmt);
+                n64_inv_store<RTW>(acc[c][0], acc[c][1], X, m, col, 2 * rr, sg, 16 * rt0 + x16, B, cpf);
         }
 }
 

@@ -302,7 +302,7 @@ __device__ __forceinline__ void naive64_inv_kc(const double* __restrict__ cre, c
             const int col = (cb * CT + (ew & (CT - 1))) * 16 + 4 * (el >> 4) + 2 * r2;
             if (col < F * cpf)
                 n64_inv_store<JT>(acc[0], acc[1], X, mm, col, 2 * r2, 1.0, 16 * (rz + (ew >> LC) * JT) + (el & 15), B,
-                                  cpf, fmt);
+                                  cpf);
         }
 #pragma unroll
         for (int i = 0; i < JT; ++i) acc[0][i] = acc[1][i] = dvec4{0.0, 0.0, 0.0, 0.0};
