@@ -105,7 +105,7 @@ def ring_fft_instance(n):
     not a power of two (the host's choice in s2_kernels.hip, fft_cfg): 1 the
     register mixed-radix passes (prime factors up to 19), else Bluestein with
     a convolution of length M >= 2n-1, 2 for a power-of-two M (taken when
-    within 5/4 of the smallest 7-smooth length), 3 for that 7-smooth M."""
+    within 5/4 of the smallest 7-smooth length), 4 for that 7-smooth M."""
     if smooth(n, 19):
         return 1
     p2 = 1
@@ -114,7 +114,7 @@ def ring_fft_instance(n):
     ms = 2 * n - 1
     while not smooth(ms, 7):
         ms += 1
-    return 2 if 4 * p2 <= 5 * ms else 3
+    return 2 if 4 * p2 <= 5 * ms else 4
 
 
 def kernels_gen(bw, form):
@@ -125,9 +125,11 @@ def kernels_gen(bw, form):
         k = KERNELS[form]
         return {"phi_fwd": f"k_phi_fwd<float2, {mode}>", "leg_fwd": k["leg_fwd"], "leg_inv": k["leg_inv"],
                 "phi_inv": f"k_phi_inv<float2, {mode}>"}
-    return {"phi_fwd": f"k_phi_fwd<double2, {mode}>", "dct_fwd": f"k_dct_fwd<double2, {mode}>",
+    # FP64 rings up to 1024 samples with a prime factor above 19: prime-factor DFTs on MFMA
+    phi = 3 if mode != 1 and bw <= 512 else mode
+    return {"phi_fwd": f"k_phi_fwd<double2, {phi}>", "dct_fwd": f"k_dct_fwd<double2, {mode}>",
             "leg_fwd": "k_gemm_fwd<double, true, CT>", "leg_inv": "k_gemm_inv<double, true, CT>",
-            "dct_inv": f"k_dct_inv<double2, {mode}>", "phi_inv": f"k_phi_inv<double2, {mode}>"}
+            "dct_inv": f"k_dct_inv<double2, {mode}>", "phi_inv": f"k_phi_inv<double2, {phi}>"}
 
 
 def kernel_map(form, bw, nfields):

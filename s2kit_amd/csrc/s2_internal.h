@@ -96,6 +96,10 @@ struct DevConsts {
     int blu_M = 0;
     double2* blu = nullptr;
     float2* blu32 = nullptr;
+    // FP64 ring DFTs by prime factors (s2_prime_dft.h): the prime above 19 of a
+    // ring length up to 1024 (else 0), its tables
+    int dft_P = 0;
+    double* dft = nullptr;
 };
 
 // Zero-padded, parity-split Legendre matrices for the MFMA GEMMs of the fast

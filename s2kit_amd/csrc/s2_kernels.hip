@@ -16,13 +16,15 @@
 // The ring FFTs of these kernels come in four instances: radix-2 Stockham
 // passes in LDS for power-of-two lengths, in-place register passes of radix
 // 2/4/8 and odd primes up to 19 for lengths with no larger prime factor, and
-// Bluestein's convolution (power-of-two or 7-smooth length) otherwise;
+// Bluestein's convolution (power-of-two or 7-smooth length) otherwise -- or,
+// for FP64 ring FFTs up to 1024 samples, the DFTs of s2_prime_dft.h;
 // power-of-two grids of 64 .. 2048 points take the register radix-8 kernels
 // of s2_blocks.h instead.  Both DCTs use one complex FFT of length N = 2B on
 // a reordered sequence (Makhoul); the DCTs are real-linear with real kernels,
 // so one complex row carries the real and imaginary transforms together.
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -147,12 +149,18 @@ __device__ __forceinline__ void dft_store(T* v, const typename Real<T>::type* cs
     }
 }
 
-// One in-place pass of radix R over nfft length-N transforms (row stride N):
+// Start of row f in LDS, rows of N values back to back.
+struct RowsOf {
+    int N;
+    __device__ __forceinline__ int operator()(int f) const { return f * N; }
+};
+
+// One in-place pass of radix R over nfft length-N transforms (row f at a + row(f)):
 // butterfly j = jq*Ns + k (k < Ns, j < N/R) reads a[j + q*N/R], applies the
 // twiddles exp(SIGN 2 pi i q k / (Ns*R)), runs an R-point DFT and writes
 // output p to a[jq*Ns*R + p*Ns + k].  tw[t] = exp(-2 pi i t / N) (in LDS).
-template <typename T, int SIGN, int R, int PER>
-__device__ __forceinline__ void mr_reg_pass(T* a, int N, int Ns, int nfft, const T* __restrict__ tw) {
+template <typename T, int SIGN, int R, int PER, typename ROW>
+__device__ __forceinline__ void mr_reg_pass(T* a, int N, int Ns, int nfft, const T* __restrict__ tw, ROW row) {
     using F = typename Real<T>::type;
     constexpr int H = (R - 1) / 2;
     const int NR = N / R, step = N / (Ns * R);
@@ -164,7 +172,7 @@ __device__ __forceinline__ void mr_reg_pass(T* a, int N, int Ns, int nfft, const
         const int bf = threadIdx.x + u * kMrThreads;
         if (bf < total) {
             const int f = div16(bf, mNR), j = bf - f * NR;
-            const T* in = a + f * N + j;
+            const T* in = a + row(f) + j;
 #pragma unroll
             for (int q = 0; q < R; ++q) v[u][q] = in[q * NR];
         }
@@ -195,7 +203,7 @@ __device__ __forceinline__ void mr_reg_pass(T* a, int N, int Ns, int nfft, const
                     v[u][q] = cmul(v[u][q], w);
                 }
             }
-            dft_store<T, SIGN, R>(v[u], cs, sn, a + f * N + jq * Ns * R + k, Ns);
+            dft_store<T, SIGN, R>(v[u], cs, sn, a + row(f) + jq * Ns * R + k, Ns);
         }
     }
     __syncthreads();
@@ -222,26 +230,26 @@ __device__ __forceinline__ int mr_reg_radix(int rem) {
     return R;
 }
 
-// In-place FFTs (natural order in and out) of nfft rows of length N, row
-// stride N, nfft*N <= rm_elems<T>(); every prime factor of N at most
+// In-place FFTs (natural order in and out) of nfft rows of length N, row f at
+// a + row(f), nfft*N <= rm_elems<T>(); every prime factor of N at most
 // PMAX (rm_supported).  One pass per radix of mr_reg_radix.
-template <typename T, int SIGN, int PMAX = kRegMaxPrime>
-__device__ __forceinline__ void mr_reg_fft(T* a, int N, int nfft, const T* __restrict__ tw) {
+template <typename T, int SIGN, int PMAX = kRegMaxPrime, typename ROW>
+__device__ __forceinline__ void mr_reg_fft(T* a, int N, int nfft, const T* __restrict__ tw, ROW row) {
     constexpr int E = rm_elems<T>();
     int rem = N, Ns = 1;
     while (rem > 1) {
         const int R = mr_reg_radix(rem);
         switch (R) {
-            case 2: mr_reg_pass<T, SIGN, 2, rm_per<E, 2>()>(a, N, Ns, nfft, tw); break;
-            case 3: mr_reg_pass<T, SIGN, 3, rm_per<E, 3>()>(a, N, Ns, nfft, tw); break;
-            case 4: mr_reg_pass<T, SIGN, 4, rm_per<E, 4>()>(a, N, Ns, nfft, tw); break;
-            case 8: mr_reg_pass<T, SIGN, 8, rm_per<E, 8>()>(a, N, Ns, nfft, tw); break;
-            case 5: mr_reg_pass<T, SIGN, 5, rm_per<E, 5>()>(a, N, Ns, nfft, tw); break;
-            case 7: mr_reg_pass<T, SIGN, 7, rm_per<E, 7>()>(a, N, Ns, nfft, tw); break;
-            case 11: if constexpr (PMAX >= 11) mr_reg_pass<T, SIGN, 11, rm_per<E, 11>()>(a, N, Ns, nfft, tw); break;
-            case 13: if constexpr (PMAX >= 13) mr_reg_pass<T, SIGN, 13, rm_per<E, 13>()>(a, N, Ns, nfft, tw); break;
-            case 17: if constexpr (PMAX >= 17) mr_reg_pass<T, SIGN, 17, rm_per<E, 17>()>(a, N, Ns, nfft, tw); break;
-            case 19: if constexpr (PMAX >= 19) mr_reg_pass<T, SIGN, 19, rm_per<E, 19>()>(a, N, Ns, nfft, tw); break;
+            case 2: mr_reg_pass<T, SIGN, 2, rm_per<E, 2>()>(a, N, Ns, nfft, tw, row); break;
+            case 3: mr_reg_pass<T, SIGN, 3, rm_per<E, 3>()>(a, N, Ns, nfft, tw, row); break;
+            case 4: mr_reg_pass<T, SIGN, 4, rm_per<E, 4>()>(a, N, Ns, nfft, tw, row); break;
+            case 8: mr_reg_pass<T, SIGN, 8, rm_per<E, 8>()>(a, N, Ns, nfft, tw, row); break;
+            case 5: mr_reg_pass<T, SIGN, 5, rm_per<E, 5>()>(a, N, Ns, nfft, tw, row); break;
+            case 7: mr_reg_pass<T, SIGN, 7, rm_per<E, 7>()>(a, N, Ns, nfft, tw, row); break;
+            case 11: if constexpr (PMAX >= 11) mr_reg_pass<T, SIGN, 11, rm_per<E, 11>()>(a, N, Ns, nfft, tw, row); break;
+            case 13: if constexpr (PMAX >= 13) mr_reg_pass<T, SIGN, 13, rm_per<E, 13>()>(a, N, Ns, nfft, tw, row); break;
+            case 17: if constexpr (PMAX >= 17) mr_reg_pass<T, SIGN, 17, rm_per<E, 17>()>(a, N, Ns, nfft, tw, row); break;
+            case 19: if constexpr (PMAX >= 19) mr_reg_pass<T, SIGN, 19, rm_per<E, 19>()>(a, N, Ns, nfft, tw, row); break;
             default: break;  // excluded on the host (rm_supported, bluestein_length)
         }
         rem /= R;
@@ -253,6 +261,11 @@ __device__ __forceinline__ void mr_reg_fft(T* a, int N, int nfft, const T* __res
 // threads in one batch).
 constexpr int kFillBatch = 4;
 
+}  // namespace s2
+
+#include "s2_prime_dft.h"
+
+namespace s2 {
 
 // nfft independent power-of-two transforms of length N stored back to back
 // in a, radix-2 Stockham passes between a and b (scratch of the same size).
@@ -351,7 +364,7 @@ __device__ __forceinline__ void bluestein_rows(T* a, int N, int M, int nfft, con
         if (blu_tw2<T>(M)) fft_block<T, -1, V, kMrThreads, true>(a, __builtin_ctz(M), S, twl);
         else fft_block<T, -1, V, kMrThreads, false>(a, __builtin_ctz(M), S, twl);
     } else {
-        mr_reg_fft<T, -1, kBluMaxPrime>(a, M, rows, twl);
+        mr_reg_fft<T, -1, kBluMaxPrime>(a, M, rows, twl, RowsOf{M});
     }
     for (int i = threadIdx.x; i < tot; i += kMrThreads) {
         const int r = div16(i, mM), k = i - r * M;
@@ -364,7 +377,7 @@ __device__ __forceinline__ void bluestein_rows(T* a, int N, int M, int nfft, con
         if (blu_tw2<T>(M)) fft_block<T, -1, V, kMrThreads, true>(a, __builtin_ctz(M), S, twl);
         else fft_block<T, -1, V, kMrThreads, false>(a, __builtin_ctz(M), S, twl);
     } else {
-        mr_reg_fft<T, -1, kBluMaxPrime>(a, M, rows, twl);
+        mr_reg_fft<T, -1, kBluMaxPrime>(a, M, rows, twl, RowsOf{M});
     }
     const unsigned long long mN = magic16(N);
     for (int i = threadIdx.x; i < nfft * N; i += kMrThreads) {
@@ -416,9 +429,10 @@ __device__ __forceinline__ const T* stage_fft_twiddles(T* b, int N, int logN, co
 
 // The FFT stage of the per-field kernels: MODE 0 radix-2 passes between two
 // buffers (power-of-two N), 1 the in-place register mixed-radix passes
-// (mr_reg_fft), 2 and 3 Bluestein with M a power of two and M of small
+// (mr_reg_fft), 2 and 4 Bluestein with M a power of two and M of small
 // primes (bluestein_rows; logN holds M, tw the LDS copy of the M twiddles,
-// gtab the global tables).  Returns the buffer holding the result.
+// gtab the global tables).  Returns the buffer holding the result.  Instance 3
+// of the FP64 ring FFTs is another algorithm (s2_prime_dft.h).
 template <typename T, int SIGN, int MODE>
 __device__ __forceinline__ T* fft_rows(T* a, T* b, int N, int logN, int pow2, int nfft, const T* __restrict__ tw,
                                        const T* __restrict__ gtab) {
@@ -426,7 +440,7 @@ __device__ __forceinline__ T* fft_rows(T* a, T* b, int N, int logN, int pow2, in
         bluestein_rows<T, SIGN, MODE == 2>(a, N, logN, nfft, tw, gtab);
         return a;
     } else if constexpr (MODE == 1) {
-        mr_reg_fft<T, SIGN>(a, N, nfft, tw);
+        mr_reg_fft<T, SIGN>(a, N, nfft, tw, RowsOf{N});
         return a;
     } else {
         return radix2_fft<T, SIGN>(a, b, N, logN, nfft, tw);
@@ -448,6 +462,9 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
                                                  T* __restrict__ X, int N, int logN, int pow2, int rpb,
                                                  const T* __restrict__ tw, int real) {
     extern __shared__ __align__(16) unsigned char smem[];
+    if constexpr (MODE == 3) {  // logN holds log2 of the runs per GEMM
+        return prime_phi_fwd(re, im, X, N, logN, rpb, tw, real, smem);
+    }
     T* a = reinterpret_cast<T*>(smem);
     const int RS = row_stride<MODE>(N, logN);
     T* b = a + lds_rows<T, MODE>(rpb, logN) * RS;
@@ -1173,6 +1190,9 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
                                                  double* __restrict__ im, int N, int logN, int pow2, int B, int rpb,
                                                  const T* __restrict__ tw, int real) {
     extern __shared__ __align__(16) unsigned char smem[];
+    if constexpr (MODE == 3) {  // logN holds log2 of the runs per GEMM
+        return prime_phi_inv(X, re, im, N, logN, B, rpb, tw, real, smem);
+    }
     T* a = reinterpret_cast<T*>(smem);
     const int RS = row_stride<MODE>(N, logN);
     T* b = a + lds_rows<T, MODE>(rpb, logN) * RS;
@@ -1493,7 +1513,7 @@ static int ilog2_exact(int n) {
 // 0 for power-of-two N (radix-2 passes, 256 threads, 2048 values per block
 // in two buffers), 1 for N whose prime factors are at most kRegMaxPrime
 // (in-place register passes, 512 threads, rm_elems<T>() values per block), 2
-// and 3 for the other N (Bluestein with a power-of-two or a 7-smooth
+// and 4 for the other N (Bluestein with a power-of-two or a 7-smooth
 // convolution length M, 512 threads, blu_rows(M) rows per block).  The
 // in-place instances also hold their twiddles in LDS.  Separate instances
 // keep each path's registers out of the others.
@@ -1534,11 +1554,11 @@ static FftCfg<T> fft_cfg(const DevConsts& c) {
     const int M = c.blu_M, rpb = blu_rows<T>(M);
     const T* g = reinterpret_cast<const T*>(f64 ? (const void*)c.blu : (const void*)c.blu32);
     const int ntw = blu_tw2<T>(M) ? tw2_values(M) : M;  // LDS twiddles
-    return {is_pow2(M) ? 2 : 3, rpb, M, sizeof(T) * ((size_t)rpb * blu_stride(M) + ntw), g};
+    return {is_pow2(M) ? 2 : 4, rpb, M, sizeof(T) * ((size_t)rpb * blu_stride(M) + ntw), g};
 }
 
 // FFT_INSTANCES(k, T): the four instances of a per-field FFT/DCT kernel.
-#define FFT_INSTANCES(k, T) k<T, 0>, k<T, 1>, k<T, 2>, k<T, 3>
+#define FFT_INSTANCES(k, T) k<T, 0>, k<T, 1>, k<T, 2>, k<T, 4>
 template <typename T, typename K0, typename K1, typename K2, typename K3, typename... A>
 static void fft_launch(const FftCfg<T>& g, K0 k0, K1 k1, K2 k2, K3 k3, dim3 grid, hipStream_t s, A... args) {
     switch (g.mode) {
@@ -1615,6 +1635,36 @@ static void bluestein_tables(int N, int& M, std::vector<double2>& out) {
     for (int k = 0; k < M; ++k) out[M + N + k] = make_double2((double)(br[k] / M), (double)(bi[k] / M));
 }
 
+// Tables of the FP64 ring DFTs of length N (s2_prime_dft.h), P the largest
+// prime factor of N.
+static void prime_tables(int N, int& P, std::vector<double>& out) {
+    P = N;
+    for (int p = 2; p < P; ++p)
+        while (P % p == 0 && P > p) P /= p;
+    const PrimeDft d = prime_dft(N, P);
+    out.assign(prime_table_doubles(d), 0.0);
+    std::memcpy(out.data(), &d, sizeof d);
+    double* tw = out.data() + 8;
+    for (int t = 0; t < d.R; ++t) {
+        tw[2 * t] = (double)cosl(2 * kPiL * t / d.R);
+        tw[2 * t + 1] = (double)-sinl(2 * kPiL * t / d.R);
+    }
+    std::vector<double> cs(P), sn(P);
+    for (int t = 0; t < P; ++t) {
+        cs[t] = (double)cosl(2 * kPiL * t / P);
+        sn[t] = (double)sinl(2 * kPiL * t / P);
+    }
+    double* tab = tw + 2 * d.R;
+    for (int ks = 0; ks < d.KS; ++ks)
+        for (int t = 0; t < d.T; ++t)
+            for (int lane = 0; lane < 64; ++lane) {
+                const int p = 16 * t + (lane & 15), k = 4 * ks + (lane >> 4);
+                double* e = tab + ((size_t)ks * 2 * d.T + t) * 64 + lane;
+                if (p <= d.H && k <= d.H) e[0] = cs[p * k % P];
+                if (p <= d.H && k < d.H) e[d.T * 64] = sn[p * (k + 1) % P];
+            }
+}
+
 void consts_create(DevConsts& c, int bw, const double* h_weights, hipStream_t s) {
     c.bw = bw;
     c.N = 2 * bw;
@@ -1685,6 +1735,12 @@ void consts_create(DevConsts& c, int bw, const double* h_weights, hipStream_t s)
         S2_HIP(hipMemcpyAsync(c.blu, blu.data(), sizeof(double2) * blu.size(), hipMemcpyHostToDevice, s));
         S2_HIP(hipMemcpyAsync(c.blu32, blu32.data(), sizeof(float2) * blu.size(), hipMemcpyHostToDevice, s));
     }
+    std::vector<double> dft;
+    if (!c.pow2 && !rm_supported(N) && N <= kPrimeMaxN) {
+        prime_tables(N, c.dft_P, dft);
+        S2_HIP(hipMalloc(&c.dft, sizeof(double) * dft.size()));
+        S2_HIP(hipMemcpyAsync(c.dft, dft.data(), sizeof(double) * dft.size(), hipMemcpyHostToDevice, s));
+    }
     S2_HIP(hipStreamSynchronize(s));  // host vectors go out of scope
     S2_HIP(hipFree(d_w));
 }
@@ -1692,7 +1748,7 @@ void consts_create(DevConsts& c, int bw, const double* h_weights, hipStream_t s)
 void consts_destroy(DevConsts& c) {
     for (void* p : {(void*)c.w_semi, (void*)c.w_naive, (void*)c.tw, (void*)c.ph, (void*)c.sinv, (void*)c.deg,
                     (void*)c.tw32, (void*)c.ph32, (void*)c.w_semi32, (void*)c.sinv32, (void*)c.trow, (void*)c.blu,
-                    (void*)c.blu32})
+                    (void*)c.blu32, (void*)c.dft})
         if (p) (void)hipFree(p);
     c = DevConsts{};
 }
@@ -1867,6 +1923,67 @@ static void reg_launch(const RegBlocks& rb, L&& launch) {
     else launch(std::integral_constant<int, kThreads>{});
 }
 
+// Rings per block of the prime-factor DFTs and log2 of their runs: the count
+// of least estimated time (cycles of a CU's blocks one after another, each its
+// MFMAs on its fullest SIMD, its memory traffic at a CU's share of the
+// bandwidth and a fixed part) whose rings stay within 80 KiB of LDS (two blocks per CU),
+// and within rm_elems where the register passes do the R-point part.
+struct PrimeCfg {
+    int nr, lr;
+    size_t lds;
+};
+static PrimeCfg prime_cfg(const PrimeDft& d, int F) {
+    const int N = d.R * d.P;
+    PrimeCfg best{1, 0, 0};
+    double bt = 0.0;
+    for (int nr = 1; nr <= N; ++nr) {
+        const size_t lds = sizeof(double2) * prime_lds_values(d, nr);
+        if (lds > 81920 || (d.R != 2 && d.R != 4 && nr * N > rm_elems<double2>())) break;
+        const int ct = (2 * nr * d.R + 15) / 16, lr = prime_runs_log2(d, ct), per = 4 >> lr;
+        const double mfma = 64.0 * d.KS * ((ct + per - 1) / per) * (2 * d.T) / (1 << lr);
+        const int blocks = (N + nr - 1) / nr * F;
+        const double t = ((blocks + 255) / 256) * (mfma + 32.0 / 9 * nr * N + 4000);
+        if (nr == 1 || t < bt) {
+            best = {nr, lr, lds};
+            bt = t;
+        }
+    }
+    return best;
+}
+
+// Ring FFTs of the per-field pipeline, power-of-two rings of the batched
+// kernels' lengths apart.  Ring lengths up to 1024 with a prime factor above
+// 19 take the prime-factor DFTs on MFMA (instance 3).
+static void ring_fft_fwd(const DevConsts& c, const FftCfg<double2>& fg, const double* re, const double* im, double2* X,
+                         int F, Fmt fmt, hipStream_t s) {
+    const int N = c.N, real = (int)(fmt == Fmt::Real);
+    if (c.dft_P) {
+        const PrimeDft d = prime_dft(N, c.dft_P);
+        const PrimeCfg g = prime_cfg(d, F);
+        launch_lds(k_phi_fwd<double2, 3>, dim3((N + g.nr - 1) / g.nr, F), kMrThreads, g.lds, s, re, im, X, N, g.lr, 0,
+                   g.nr, (const double2*)c.dft, real);
+    } else {
+        fft_launch(fg, FFT_INSTANCES(k_phi_fwd, double2), dim3((N + fg.rpb - 1) / fg.rpb, F), s, re, im, X, N, fg.lg,
+                   c.pow2, fg.rpb, fg.tw, real);
+    }
+    S2_HIP(hipGetLastError());
+}
+
+static void ring_fft_inv(const DevConsts& c, const FftCfg<double2>& fg, const double2* X, double* re, double* im, int F,
+                         Fmt fmt, hipStream_t s) {
+    const int N = c.N, B = c.bw, real = (int)(fmt == Fmt::Real);
+    if (c.dft_P) {
+        const PrimeDft d = prime_dft(N, c.dft_P);
+        const PrimeCfg g = prime_cfg(d, F);
+        launch_lds(k_phi_inv<double2, 3>, dim3((N + g.nr - 1) / g.nr, F), kMrThreads, g.lds, s, X, re, im, N, g.lr, 0,
+                   B, g.nr, (const double2*)c.dft, real);
+    } else {
+        fft_launch(fg, FFT_INSTANCES(k_phi_inv, double2), dim3((N + fg.rpb - 1) / fg.rpb, F), s, X, re, im, N, fg.lg,
+                   c.pow2, B, fg.rpb, fg.tw, real);
+    }
+    S2_HIP(hipGetLastError());
+}
+
 // FP32 ring FFTs of grids whose ring length is not a power of two (the mixed
 // form's first and last stages at such bandwidths), on the register
 // mixed-radix or Bluestein instances; same order-major FP32 intermediate X
@@ -1904,8 +2021,7 @@ void forward_fp64(const DevConsts& c, const DevTables& t, const double* re, cons
                        X, c.logN, c.tw, f);
         });
     else
-        fft_launch(fg, FFT_INSTANCES(k_phi_fwd, double2), dim3((N + rpb - 1) / rpb, F),
-                   s, re, im, X, N, fg.lg, c.pow2, rpb, fg.tw, (int)(fmt == Fmt::Real));
+        ring_fft_fwd(c, fg, re, im, X, F, fmt, s);
     S2_HIP(hipGetLastError());
     }
     if (cut > 0) {
@@ -2012,8 +2128,7 @@ void inverse_fp64(const DevConsts& c, const DevTables& t, const double* cre, con
                        (const double2*)X, re, im, c.logN, c.tw, f);
         });
     else
-        fft_launch(fg, FFT_INSTANCES(k_phi_inv, double2), dim3((N + rpb - 1) / rpb, F),
-                   s, X, re, im, N, fg.lg, c.pow2, B, rpb, fg.tw, (int)(fmt == Fmt::Real));
+        ring_fft_inv(c, fg, X, re, im, F, fmt, s);
     S2_HIP(hipGetLastError());
 }
 
@@ -2025,9 +2140,7 @@ void forward_fp64_gemm(const DevConsts& c, const GemmTables& g, const double* re
     const int rpb = fg.rpb;
     {
         Span sp(tm, ST_PHI_FWD, s);
-        fft_launch(fg, FFT_INSTANCES(k_phi_fwd, double2), dim3((N + rpb - 1) / rpb, F),
-                   s, re, im, X, N, fg.lg, c.pow2, rpb, fg.tw, (int)(fmt == Fmt::Real));
-        S2_HIP(hipGetLastError());
+        ring_fft_fwd(c, fg, re, im, X, F, fmt, s);
     }
     if (cut > 0) {
         const int nrows = (fmt == Fmt::Complex) ? 2 * cut - 1 : cut;
@@ -2058,9 +2171,7 @@ void inverse_fp64_gemm(const DevConsts& c, const GemmTables& g, const double* cr
         S2_HIP(hipGetLastError());
     }
     Span sp(tm, ST_PHI_INV, s);
-    fft_launch(fg, FFT_INSTANCES(k_phi_inv, double2), dim3((N + rpb - 1) / rpb, F), s,
-               X, re, im, N, fg.lg, c.pow2, B, rpb, fg.tw, (int)(fmt == Fmt::Real));
-    S2_HIP(hipGetLastError());
+    ring_fft_inv(c, fg, X, re, im, F, fmt, s);
 }
 
 void zonal_fp64(const DevConsts& c, const DevTables& t, const double* re, const double* im, double* zr, double* zi,

@@ -9,6 +9,8 @@ Mixed plans (FP32 FFTs + naive DLT on FP32 MFMA): 1e-6, at power-of-two
 bandwidths and others (mixed-radix FP32 FFTs, GEMMs over rings padded to
 whole 64-ring groups).
 """
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -577,3 +579,70 @@ def test_dense_fp64_legendre(env, O, bw, F, cutoff, fmt):
             one.forward(gre[f:f + 1], gim[f:f + 1], a, b, data_format=fmt)
             assert torch.equal(a, c2r[f:f + 1]) and torch.equal(b, c2i[f:f + 1])
     one.close()
+
+
+@pytest.mark.parametrize("bw,F", [
+    (23, 1), (23, 70), (37, 9), (46, 30), (58, 2), (69, 25), (92, 3), (101, 40), (127, 1), (131, 17), (202, 5), (251, 4),
+    (253, 9), (257, 2), (263, 3), (303, 4), (437, 2), (509, 1), (511, 3)])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_prime_factor_ring_ffts(env, O, bw, F, fmt):
+    # FP64 ring lengths with a prime factor P above 19: one and several row
+    # tiles per wave (P = 23 to 509), the R-point parts 2, 4, powers of two and
+    # odd multiples (up to R = 38), last blocks with fewer rings, few and many
+    # fields (the rings per block follow the call's size).  A REAL analysis
+    # ignores no imaginary sample (both planes hold data here).
+    S, torch, dev = env
+    n = 2 * bw
+    print(f"prime-factor rings bw={bw} F={F} fmt={fmt}", flush=True)
+    ends = sorted({0, F - 1})
+    coeffs = {f: O.make_coeffs(700 + f, bw, 2 if fmt == 1 else 0) for f in ends}
+    cre = to_dev(torch, dev, [coeffs.get(f, coeffs[0])[0] for f in range(F)])
+    cim = to_dev(torch, dev, [coeffs.get(f, coeffs[0])[1] for f in range(F)])
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(bw)
+    hre, him = (torch.randn((F, n, n), generator=gen, dtype=torch.float64, device=dev) for _ in range(2))
+    gre, gim = torch.empty_like(hre), torch.empty_like(hre)
+    c2r, c2i = torch.empty_like(cre), torch.empty_like(cim)
+    with contextlib.closing(S.Plan(bw, F, precision=0)) as plan:
+        plan.inverse(cre, cim, gre, gim, data_format=fmt)
+        plan.forward(hre, him, c2r, c2i, data_format=fmt)
+        torch.cuda.synchronize()
+    for f in ends:
+        og = O.inv_fst(coeffs[f][0], coeffs[f][1], bw, data_format=fmt)
+        assert crel(gre[f].cpu().numpy().ravel(), gim[f].cpu().numpy().ravel(), *og) < 1e-11
+        oc = O.fst(hre[f].cpu().numpy().ravel(), him[f].cpu().numpy().ravel(), bw, data_format=fmt)
+        assert crel(c2r[f].cpu().numpy(), c2i[f].cpu().numpy(), *oc) < 1e-11
+
+
+@pytest.mark.parametrize("bw,F,prec,tol", [
+    (64, 1, 0, 1e-12), (64, 9, 0, 1e-12), (100, 5, 0, 1e-12), (131, 2, 0, 1e-12), (600, 1, 0, 1e-11), (128, 65, 1, 1e-4),
+    (32, 3, 2, 1e-5), (128, 65, 2, 1e-5), (100, 5, 2, 1e-5), (131, 2, 2, 1e-5), (64, 9, 3, 1e-5)])
+def test_real_format_matches_complex(env, bw, F, prec, tol):
+    # REAL calls read and write the order rows m < bw only; on Hermitian
+    # coefficients and real samples they agree with COMPLEX calls.
+    S, torch, dev = env
+    n = 2 * bw
+    print(f"real format bw={bw} F={F} prec={prec}", flush=True)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(bw)
+    g = torch.randn((F, n, n), generator=gen, dtype=torch.float64, device=dev)
+    z = torch.zeros_like(g)
+
+    def rel(x, y):
+        return float((x - y).norm() / y.norm())
+
+    with contextlib.closing(S.Plan(bw, F, precision=prec)) as plan:
+        out = {}
+        for fmt in (0, 1):
+            a, b = (torch.empty((F, bw * bw), dtype=torch.float64, device=dev) for _ in range(2))
+            plan.forward(g, z, a, b, data_format=fmt)
+            out[fmt] = torch.complex(a, b)
+        assert rel(out[1], out[0]) < tol
+        cre, cim = out[1].real.contiguous(), out[1].imag.contiguous()
+        syn = {}
+        for fmt in (0, 1):
+            x, y = torch.empty_like(g), torch.empty_like(g)
+            plan.inverse(cre, cim, x, y, data_format=fmt)
+            syn[fmt] = x
+        torch.cuda.synchronize()
+        assert rel(syn[1], syn[0]) < tol
