@@ -572,12 +572,10 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
 }
 
 // Seminaive projections of orders m < cut.  grid (cut, ceil(F/fc)); block m
-// handles rows m and N-m of fc fields.  zonal: write only degree l of order 0
-// into zr/zi [F][B] (FZTSemiMemo).
+// handles rows m and N-m of fc fields.
 __global__ __launch_bounds__(256) void k_leg_fwd(const double2* __restrict__ Cb, const double* __restrict__ T,
                                                  const long* __restrict__ toff, double* __restrict__ cre,
-                                                 double* __restrict__ cim, int N, int B, int F, int fc, int fmt,
-                                                 int zonal) {
+                                                 double* __restrict__ cim, int N, int B, int F, int fc, int fmt) {
     extern __shared__ __align__(16) unsigned char smem[];
     double2* cs = reinterpret_cast<double2*>(smem);
     const int m = blockIdx.x, f0 = blockIdx.y * fc;
@@ -607,10 +605,7 @@ __global__ __launch_bounds__(256) void k_leg_fwd(const double2* __restrict__ Cb,
             ai += cv.y * tv;
         }
         const int f = f0 + fl;
-        if (zonal) {
-            cre[(size_t)f * B + l] = ar;
-            cim[(size_t)f * B + l] = (fmt == 0) ? ai : 0.0;
-        } else if (s == 0) {
+        if (s == 0) {
             const int p = index_of_coeff(m, l, B);
             cre[f * B2 + p] = ar;
             cim[f * B2 + p] = ai;
@@ -626,6 +621,69 @@ __global__ __launch_bounds__(256) void k_leg_fwd(const double2* __restrict__ Cb,
         }
     }
 }
+
+// Zonal projections (FZTSemiMemo): degree l of order 0 of every field, into
+// zr/zi [F][B], from row 0's cosine coefficients and the order's table T.  A
+// block takes kZonalL degrees of kZonalF fields, a thread each, kZonalT terms at
+// a time staged in LDS: table rows are read along their length (a thread per row
+// walking its own row touched a line per lane and term).  Each sum keeps the
+// ascending order of k_leg_fwd.  Bound by latency: few blocks of a short serial
+// chain, so four fields per block, and every load of a step issued before its
+// first LDS store (conditional loads, each waited for at its store: 30 us at bw=512).
+// Measured against k_leg_fwd's one block per 65536 / 32 B fields: bw=512
+// x25 67 -> 9.7 us, bw=256 x76 50 -> 6.2, bw=64 x153 22 -> 4.0.
+// grid (ceil(B/kZonalL), ceil(F/kZonalF)).
+constexpr int kZonalL = 32, kZonalF = 4, kZonalT = 64;
+__global__ __launch_bounds__(kZonalL * kZonalF) void k_zonal(const double2* __restrict__ Cb, const double* __restrict__ T,
+                                                             double* __restrict__ zr, double* __restrict__ zi, int N,
+                                                             int B, int F, int fmt) {
+    constexpr int NTH = kZonalL * kZonalF;
+    __shared__ double tile[kZonalL][kZonalT + 1];
+    __shared__ double2 cs[kZonalF][2 * kZonalT + 1];
+    const int l0 = blockIdx.x * kZonalL, f0 = blockIdx.y * kZonalF;
+    const int dl = threadIdx.x % kZonalL, fl = threadIdx.x / kZonalL, l = l0 + dl;
+    const int rs = l < B ? row_size(0, l) : 0, rsmax = row_size(0, min(l0 + kZonalL, B) - 1);
+    constexpr int NR = kZonalL * kZonalT / NTH;  // table loads per thread and step
+    const int r0 = threadIdx.x / kZonalT, tt = threadIdx.x % kZonalT;
+    double ar = 0.0, ai = 0.0;
+    for (int t0 = 0; t0 < rsmax; t0 += kZonalT) {
+        // all loads first (past the last row, term or field they repeat it)
+        double tv[NR];
+        double2 cv[kZonalF];
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            const int lr = min(l0 + r0 + u * (NTH / kZonalT), B - 1);
+            tv[u] = T[table_offset(0, lr) + min(t0 + tt, row_size(0, lr) - 1)];
+        }
+#pragma unroll
+        for (int f = 0; f < kZonalF; ++f)
+            cv[f] = Cb[(size_t)min(f0 + f, F - 1) * N * B + min(2 * t0 + (int)threadIdx.x, B - 1)];
+#pragma unroll
+        for (int u = 0; u < NR; ++u) tile[r0 + u * (NTH / kZonalT)][tt] = tv[u];
+#pragma unroll
+        for (int f = 0; f < kZonalF; ++f) cs[f][threadIdx.x] = cv[f];
+        __syncthreads();
+        const int nt = min(kZonalT, rs - t0);
+        auto term = [&](int t) __attribute__((always_inline)) {
+            const double tv = tile[dl][t];
+            const double2 cv = cs[fl][2 * t + (l & 1)];
+            ar += cv.x * tv;
+            ai += cv.y * tv;
+        };
+        int t = 0;
+        for (; t + 8 <= nt; t += 8) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) term(t + e);
+        }
+        for (; t < nt; ++t) term(t);
+        __syncthreads();
+    }
+    if (l < B && f0 + fl < F) {
+        zr[(size_t)(f0 + fl) * B + l] = ar;
+        zi[(size_t)(f0 + fl) * B + l] = (fmt == 0) ? ai : 0.0;
+    }
+}
+static_assert(kZonalL * kZonalF == 2 * kZonalT && kZonalL * kZonalF % kZonalT == 0, "k_zonal's loads");
 
 // Naive projections of orders m >= cut (DLTNaive: even weights for every
 // order).  grid (B-cut, ceil(F/fc)).  w_naive = even weights * sqrt(2pi)/N.
@@ -1239,6 +1297,9 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
 
 // m = 0 bin of each ring as a direct sum (FST_semi_memo.c:386-398), into
 // row 0 of X.  One wavefront per ring; grid (ceil(N/4), F), block 256.
+// Bound by the read of the grids: the loads are marked non-temporal and eight
+// per lane and plane are in flight (bw=512 x 25, 419 MB: 118 -> 85 us with eight
+// in flight -> 62 us non-temporal; bw=256 x 76, 319 MB: 110 -> 84 -> 46 us).
 __global__ __launch_bounds__(256) void k_ring_sum(const double* __restrict__ re, const double* __restrict__ im,
                                                   double2* __restrict__ X, int N) {
     const int f = blockIdx.y;
@@ -1247,9 +1308,21 @@ __global__ __launch_bounds__(256) void k_ring_sum(const double* __restrict__ re,
     if (j >= N) return;
     const size_t base = ((size_t)f * N + j) * N;
     double sr = 0.0, si = 0.0;
-    for (int k = lane; k < N; k += 64) {
-        sr += re[base + k];
-        si += im[base + k];
+    constexpr int U = 8;
+    for (int k0 = lane; k0 < N; k0 += 64 * U) {
+        double a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + 64 * u < N) {
+                a[u] = __builtin_nontemporal_load(re + base + k0 + 64 * u);
+                b[u] = __builtin_nontemporal_load(im + base + k0 + 64 * u);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + 64 * u < N) {
+                sr += a[u];
+                si += b[u];
+            }
     }
     for (int o = 32; o > 0; o >>= 1) {
         sr += __shfl_xor(sr, o);
@@ -2060,7 +2133,7 @@ void forward_fp64(const DevConsts& c, const DevTables& t, const double* re, cons
         } else {
             const int fc = std::max(1, 65536 / (2 * B * (int)sizeof(double2)));
             k_leg_fwd<<<dim3(cut, (F + fc - 1) / fc), 256, sizeof(double2) * 2 * B * std::min(fc, F), s>>>(
-                Cb, t.fwd, t.off, cre, cim, N, B, F, fc, f, 0);
+                Cb, t.fwd, t.off, cre, cim, N, B, F, fc, f);
         }
         S2_HIP(hipGetLastError());
     }
@@ -2186,9 +2259,8 @@ void zonal_fp64(const DevConsts& c, const DevTables& t, const double* re, const 
     fft_launch(fg, FFT_INSTANCES(k_dct_fwd, double2), dim3(1, F), s, X, Cb, c.w_semi,
                fg.tw, c.ph, N, fg.lg, c.pow2, B, t.cutoff, 1, 1, 0);
     S2_HIP(hipGetLastError());
-    const int fc = std::max(1, 65536 / (2 * B * (int)sizeof(double2)));
-    k_leg_fwd<<<dim3(1, (F + fc - 1) / fc), 256, sizeof(double2) * 2 * B * std::min(fc, F), s>>>(
-        Cb, t.fwd, t.off, zr, zi, N, B, F, fc, (int)fmt, 1);
+    const dim3 grid((B + kZonalL - 1) / kZonalL, (F + kZonalF - 1) / kZonalF);
+    k_zonal<<<grid, kZonalL * kZonalF, 0, s>>>(Cb, t.fwd + t.h_off.at(0), zr, zi, N, B, F, (int)fmt);
     S2_HIP(hipGetLastError());
 }
 

@@ -646,3 +646,24 @@ def test_real_format_matches_complex(env, bw, F, prec, tol):
             syn[fmt] = x
         torch.cuda.synchronize()
         assert rel(syn[1], syn[0]) < tol
+
+
+@pytest.mark.parametrize("bw,F", [(2, 1), (16, 4), (33, 5), (130, 3), (260, 9)])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_zonal_edges(env, O, bw, F, fmt):
+    # The zonal projections at the edges of their blocks (32 degrees, 4 fields)
+    # and of their steps of 64 terms (rows of more than 64 and 128 terms above
+    # bw = 128 and 256), and the ring sums' batches of eight loads.
+    S, torch, dev = env
+    n = 2 * bw
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(bw)
+    hre, him = (torch.randn((F, n, n), generator=gen, dtype=torch.float64, device=dev) for _ in range(2))
+    zr = torch.empty((F, bw), dtype=torch.float64, device=dev)
+    zi = torch.empty_like(zr)
+    with contextlib.closing(S.Plan(bw, F)) as plan:
+        plan.zonal(hre, him, zr, zi, data_format=fmt)
+        torch.cuda.synchronize()
+    for f in range(F):
+        orr, oir = O.fzt(hre[f].cpu().numpy(), him[f].cpu().numpy(), bw, data_format=fmt)
+        assert crel(zr[f].cpu().numpy(), zi[f].cpu().numpy(), orr, oir) < 1e-11
