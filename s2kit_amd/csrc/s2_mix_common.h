@@ -26,19 +26,44 @@ constexpr int kMixCols = 16 * S2_MIX_WAVES;
 // 16-degree tiles per parity of order m (the even parity has the most degrees).
 __host__ __device__ inline int mix_n0(int m, int B) { return (gm_lp(m, 0, B) + 15) / 16; }
 
-// Workgroup id -> an order pair (m, bw-1-m) and a column block cb of nb per
-// order.  A workgroup runs both orders of its pair, so every workgroup has
-// about the same work (bw-m + m+1 degrees): blocks of very different lengths
-// would leave the dispatcher's round-robin placement unbalanced.  Ids go
-// round-robin over the 8 XCDs (id mod 8); XCD k takes the pairs m = 8q+k, all
-// column blocks of one pair back to back, so the pair's table tiles stay in
-// that XCD's L2.  bw % 16 == 0.
-__device__ __forceinline__ void mix_pair(int nb, int& m, int& cb) {  // grid: mix_npairs8(bw) * nb
-    const int id = blockIdx.x, k = id & 7, local = id >> 3;
+// Data columns of order m: (field, +m or -m row, re or im), cpf per field.
+__host__ __device__ inline int mix_cpf(int m, int fmt) { return (m > 0 && fmt == 0) ? 4 : 2; }
+
+// Workgroup id -> an order pair (m, bw-1-m), the halves of it to run (h0 <= h
+// < h1; 0: order m, 1: its partner) and a column block cb of nb per order.  A
+// workgroup runs both orders of its pair, so every workgroup has about the
+// same work (bw-m + m+1 degrees): blocks of very different lengths would leave
+// the dispatcher's round-robin placement unbalanced.  With `single` (launches
+// of few blocks, mix_single) a workgroup runs one order, all orders m < bw/2, the
+// long ones, first.  Ids go round-robin over the 8 XCDs (id mod 8); XCD k takes
+// the pairs m = 8q+k, all column blocks of one pair back to back, so the pair's
+// table tiles stay in that XCD's L2.  bw % 16 == 0.
+__device__ __forceinline__ void mix_pair(int id, int nb, int& m, int& cb) {
+    const int k = id & 7, local = id >> 3;
     const int q = local / nb;
     cb = local - q * nb;
     m = 8 * q + k;  // < bw/2; its partner is bw-1-m
 }
+__device__ __forceinline__ void mix_pair(int nb, int& m, int& cb) {  // grid: mix_npairs8(bw) * nb
+    mix_pair(blockIdx.x, nb, m, cb);
+}
+__device__ __forceinline__ void mix_pair(int nb, int single, int& m, int& cb, int& h0, int& h1) {  // grid: the above << single
+    const int half = gridDim.x >> 1, hi = single && (int)blockIdx.x >= half;
+    mix_pair((int)blockIdx.x - (hi ? half : 0), nb, m, cb);
+    h0 = hi;
+    h1 = single ? h0 + 1 : 2;
+}
+// One order per workgroup for launches of fewer than 512 pair workgroups (two
+// per CU), which otherwise leave each CU one long chain of steps.  Forward / inverse GEMM,
+// us, pairs -> orders: mixed bw=64 x32 11.4 / 11.1 -> 8.2 / 9.2, bw=256 x8 41 / 34
+// -> 31 / 30, bw=256 x76 REAL 80 / 65 -> 65 / 56, bw=512 x4 116 -> 106; split
+// bw=256 x8 35 / 31 -> 26 / 25.  At 512 workgroups it lost (mixed bw=512 x16 inverse 114 ->
+// 130, split bw=256 x64 75 / 76 -> 79 / 79) or changed nothing, above as well.
+inline int mix_single(int blocks) { return blocks < 512; }
+// Column blocks of a launch; counted for the format, so that none is empty but
+// order 0's (with the COMPLEX count, every second block of a REAL call was, and
+// the placement uneven: mixed bw=512 x25 REAL 185 / 179 -> 129 / 106 us).
+inline int mix_blocks(int F, Fmt fmt) { return (mix_cpf(1, (int)fmt) * F + kMixCols - 1) / kMixCols; }
 
 // Folded rings the mixed form's GEMMs run over: bw rounded up to whole
 // 64-ring groups (32 at bw = 32); the tables are zero past bw, and the
@@ -59,9 +84,6 @@ template <int GJ>
 __host__ __device__ constexpr int mix_jt() {
     return GJ ? 4 * GJ : 2;
 }
-
-// Data columns of order m: (field, +m or -m row, re or im), cpf per field.
-__host__ __device__ inline int mix_cpf(int m, int fmt) { return (m > 0 && fmt == 0) ? 4 : 2; }
 
 typedef double dpair8 __attribute__((ext_vector_type(2))) __attribute__((aligned(8)));
 

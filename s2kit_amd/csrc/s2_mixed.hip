@@ -226,13 +226,13 @@ __device__ __forceinline__ void mix_fwd_body(const float2* __restrict__ X, const
 template <int MAXN0>
 __global__ __launch_bounds__(kMixThreads) __attribute__((amdgpu_waves_per_eu(MAXN0 > 8 ? 2 : S2_MIX_WPE_FWD))) void k_mix_fwd(const float2* __restrict__ X, const float* __restrict__ NF,
                                                         const GemmMeta* __restrict__ meta, double* __restrict__ cre,
-                                                        double* __restrict__ cim, int B, int F, int fmt, int nb) {
+                                                        double* __restrict__ cim, int B, int F, int fmt, int nb, int single) {
     extern __shared__ __align__(16) unsigned char smem[];
     float* sm = reinterpret_cast<float*>(smem);
-    int mp, cb;
-    mix_pair(nb, mp, cb);
+    int mp, cb, h0, h1;
+    mix_pair(nb, single, mp, cb, h0, h1);
     if (mp >= mix_npairs(B)) return;
-    for (int h = 0; h < 2; ++h) {
+    for (int h = h0; h < h1; ++h) {
         if (h && B - 1 - mp == mp) break;  // odd bw: the middle order pairs with itself
         const int m = h ? B - 1 - mp : mp;
         const GemmMeta g0 = meta[m * 2], g1 = meta[m * 2 + 1];
@@ -400,14 +400,15 @@ __device__ __forceinline__ void mix_inv_body(const double* __restrict__ cre, con
 template <int GJ>
 __global__ __launch_bounds__(kMixThreads) __attribute__((amdgpu_waves_per_eu(S2_MIX_WPE_INV))) void k_mix_inv(
     const double* __restrict__ cre, const double* __restrict__ cim, const float* __restrict__ NI,
-    const GemmMeta* __restrict__ meta, float2* __restrict__ X, int B, int F, int fmt, int nb) {
+    const GemmMeta* __restrict__ meta, float2* __restrict__ X, int B, int F, int fmt, int nb, int single) {
     extern __shared__ __align__(16) unsigned char smem[];
     float* sm = reinterpret_cast<float*>(smem);
-    int mp, cz;
-    mix_pair(nb * (mix_bp(B) / mix_jw<GJ>()), mp, cz);
+    int mp, cz, h0, h1;
+    mix_pair(nb * (mix_bp(B) / mix_jw<GJ>()), single, mp, cz, h0, h1);
     if (mp >= mix_npairs(B)) return;
-    mix_inv_body<GJ>(cre, cim, NI, meta, X, B, F, fmt, mp, cz, sm);
-    if (B - 1 - mp == mp) return;  // odd bw: the middle order pairs with itself
+    // (one loop over both orders spilled 15 VGPRs: bw=256 x 1024 862 -> 900 us)
+    if (h0 == 0) mix_inv_body<GJ>(cre, cim, NI, meta, X, B, F, fmt, mp, cz, sm);
+    if (h1 == 1 || B - 1 - mp == mp) return;  // odd bw: the middle order pairs with itself
     __syncthreads();  // the partner order's prologue reuses the table buffers
     mix_inv_body<GJ>(cre, cim, NI, meta, X, B, F, fmt, B - 1 - mp, cz, sm);
 }
@@ -477,20 +478,21 @@ static size_t mix_fwd_lds(int B) {
 static void mix_fwd_gemm(const DevConsts& c, const GemmTables& g, const float2* X, double* cre, double* cim, int F,
                          Fmt fmt, hipStream_t s) {
     const int B = c.bw;
-    const int nb = (4 * F + kMixCols - 1) / kMixCols;
-    const dim3 grid(mix_npairs8(B) * nb);  // order pairs x column blocks
+    const int nb = mix_blocks(F, fmt);
+    const int single = mix_single(mix_npairs8(B) * nb);
+    const dim3 grid(mix_npairs8(B) * nb << single);  // order pairs (orders) x column blocks
     const size_t lds = mix_fwd_lds(B);
     const float* nf = (const float*)g.af;
     const GemmMeta* meta = g.meta;
     const int n0max = mix_n0(0, B);
     if (n0max <= 2)
-        launch_lds(k_mix_fwd<2>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb);
+        launch_lds(k_mix_fwd<2>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb, single);
     else if (n0max <= 4)
-        launch_lds(k_mix_fwd<4>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb);
+        launch_lds(k_mix_fwd<4>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb, single);
     else if (n0max <= 8)
-        launch_lds(k_mix_fwd<8>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb);
+        launch_lds(k_mix_fwd<8>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb, single);
     else
-        launch_lds(k_mix_fwd<16>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb);
+        launch_lds(k_mix_fwd<16>, grid, kMixThreads, lds, s, X, nf, meta, cre, cim, B, F, (int)fmt, nb, single);
 }
 
 static void mix_inv_gemm(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, float2* X,
@@ -498,16 +500,18 @@ static void mix_inv_gemm(const DevConsts& c, const GemmTables& g, const double* 
     const int B = c.bw;
     const int gj = B <= 32 ? 0 : g.t_gj ? g.t_gj : mix_gj_default(B);
     const int jw = gj ? 64 * gj : 32;
-    const int nb = (4 * F + kMixCols - 1) / kMixCols;
-    const dim3 grid(mix_npairs8(B) * nb * (mix_bp(B) / jw));  // order pairs x column blocks x ring ranges
+    const int nb = mix_blocks(F, fmt);
+    const int pairs = mix_npairs8(B) * nb * (mix_bp(B) / jw);
+    const int single = mix_single(pairs);
+    const dim3 grid(pairs << single);  // order pairs (orders) x column blocks x ring ranges
     const size_t lds = sizeof(float) * 2 * (2 * kMixInvKC * jw);
     const float* ni = (const float*)g.ai;
     const GemmMeta* meta = g.meta;
     switch (gj) {
-        case 0: launch_lds(k_mix_inv<0>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb); break;
-        case 1: launch_lds(k_mix_inv<1>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb); break;
-        case 2: launch_lds(k_mix_inv<2>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb); break;
-        default: launch_lds(k_mix_inv<4>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb); break;
+        case 0: launch_lds(k_mix_inv<0>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb, single); break;
+        case 1: launch_lds(k_mix_inv<1>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb, single); break;
+        case 2: launch_lds(k_mix_inv<2>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb, single); break;
+        default: launch_lds(k_mix_inv<4>, grid, kMixThreads, lds, s, cre, cim, ni, meta, X, B, F, (int)fmt, nb, single); break;
     }
 }
 

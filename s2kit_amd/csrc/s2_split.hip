@@ -298,13 +298,13 @@ __device__ __forceinline__ void split_fwd_body(const float2* __restrict__ X, con
 template <int MAXN0>
 __global__ __launch_bounds__(kMixThreads) __attribute__((amdgpu_waves_per_eu(S2_SPLIT_WPE_FWD))) void k_split_fwd(const float2* __restrict__ X, const __bf16* __restrict__ SF,
                                                            const GemmMeta* __restrict__ meta, double* __restrict__ cre,
-                                                           double* __restrict__ cim, int lgB, int F, int fmt, int nbw) {
+                                                           double* __restrict__ cim, int lgB, int F, int fmt, int nbw, int single) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int B = 1 << lgB;
-    int mp, cw;
-    mix_pair(nbw, mp, cw);
+    int mp, cw, h0, h1;
+    mix_pair(nbw, single, mp, cw, h0, h1);
     const int cb0 = cw * kSplitBlocks;
-    for (int h = 0; h < 2; ++h) {
+    for (int h = h0; h < h1; ++h) {
         const int m = h ? B - 1 - mp : mp;
         const GemmMeta g0 = meta[m * 2];
 #define S2_SPLIT_FWD(n)                                                                                        \
@@ -462,14 +462,16 @@ __global__ __launch_bounds__(kMixThreads) __attribute__((amdgpu_waves_per_eu(S2_
                                                            const double* __restrict__ cim,
                                                            const __bf16* __restrict__ SI,
                                                            const GemmMeta* __restrict__ meta, float2* __restrict__ X,
-                                                           int lgB, int F, int fmt, int nbw) {
+                                                           int lgB, int F, int fmt, int nbw, int single) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int B = 1 << lgB;
     const int nz = B / mix_jw<GJ>();
-    int mp, cz;
-    mix_pair(nbw * nz, mp, cz);
+    int mp, cz, h0, h1;
+    mix_pair(nbw * nz, single, mp, cz, h0, h1);
     const int cw = cz / nz, jr = cz - cw * nz;
-    split_inv_body<GJ>(cre, cim, SI, meta, X, B, F, fmt, mp, cw * kSplitBlocks, kSplitBlocks, jr, smem);
+    if (h0 == 0)
+        split_inv_body<GJ>(cre, cim, SI, meta, X, B, F, fmt, mp, cw * kSplitBlocks, kSplitBlocks, jr, smem);
+    if (h1 == 1) return;
     __syncthreads();  // the partner order's first stage reuses the buffers
     split_inv_body<GJ>(cre, cim, SI, meta, X, B, F, fmt, B - 1 - mp, cw * kSplitBlocks, kSplitBlocks, jr, smem);
 }
@@ -518,21 +520,22 @@ void split_tables_create(GemmTables& g, const DevConsts& c, hipStream_t s) {
 void split_fwd_gemm(const DevConsts& c, const GemmTables& g, const float2* X, double* cre, double* cim, int F,
                     Fmt fmt, hipStream_t s) {
     const int B = c.bw;
-    const int nb = (4 * F + kMixCols - 1) / kMixCols;
+    const int nb = mix_blocks(F, fmt);
     const int nbw = (nb + kSplitBlocks - 1) / kSplitBlocks;
-    const dim3 grid(B / 2 * nbw);  // order pairs x groups of column blocks
+    const int single = mix_single(B / 2 * nbw);
+    const dim3 grid(B / 2 * nbw << single);  // order pairs (orders) x groups of column blocks
     const int n0max = mix_n0(0, B);
     const size_t lds = 2 * kSplitStage;
     const __bf16* sf = (const __bf16*)g.af;
     const GemmMeta* meta = g.meta;
     if (n0max <= 2)
-        launch_lds(k_split_fwd<2>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw);
+        launch_lds(k_split_fwd<2>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw, single);
     else if (n0max <= 4)
-        launch_lds(k_split_fwd<4>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw);
+        launch_lds(k_split_fwd<4>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw, single);
     else if (n0max <= 8)
-        launch_lds(k_split_fwd<8>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw);
+        launch_lds(k_split_fwd<8>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw, single);
     else
-        launch_lds(k_split_fwd<16>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw);
+        launch_lds(k_split_fwd<16>, grid, kMixThreads, lds, s, X, sf, meta, cre, cim, lg2(B), F, (int)fmt, nbw, single);
 }
 
 void split_inv_gemm(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, float2* X, int F,
@@ -540,17 +543,18 @@ void split_inv_gemm(const DevConsts& c, const GemmTables& g, const double* cre, 
     const int B = c.bw;
     const int gj = B < 64 ? 0 : std::min(S2_SPLIT_GJMAX, B / 64);
     const int jw = gj ? 64 * gj : 32, jt = jw / 16;
-    const int nb = (4 * F + kMixCols - 1) / kMixCols;
+    const int nb = mix_blocks(F, fmt);
     const int nbw = (nb + kSplitBlocks - 1) / kSplitBlocks;
-    const dim3 grid(B / 2 * nbw * (B / jw));  // order pairs x groups of column blocks x ring ranges
+    const int pairs = B / 2 * nbw * (B / jw), single = mix_single(pairs);
+    const dim3 grid(pairs << single);  // order pairs (orders) x groups of column blocks x ring ranges
     const size_t lds = 2 * (size_t)std::min(jt, kSplitStageTiles) * kSplitTile;
     const __bf16* si = (const __bf16*)g.ai;
     const GemmMeta* meta = g.meta;
     switch (gj) {
-        case 0: launch_lds(k_split_inv<0>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw); break;
-        case 1: launch_lds(k_split_inv<1>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw); break;
-        case 2: launch_lds(k_split_inv<2>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw); break;
-        default: launch_lds(k_split_inv<4>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw); break;
+        case 0: launch_lds(k_split_inv<0>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw, single); break;
+        case 1: launch_lds(k_split_inv<1>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw, single); break;
+        case 2: launch_lds(k_split_inv<2>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw, single); break;
+        default: launch_lds(k_split_inv<4>, grid, kMixThreads, lds, s, cre, cim, si, meta, X, lg2(B), F, (int)fmt, nbw, single); break;
     }
 }
 

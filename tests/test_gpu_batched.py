@@ -667,3 +667,30 @@ def test_zonal_edges(env, O, bw, F, fmt):
     for f in range(F):
         orr, oir = O.fzt(hre[f].cpu().numpy(), him[f].cpu().numpy(), bw, data_format=fmt)
         assert crel(zr[f].cpu().numpy(), zi[f].cpu().numpy(), orr, oir) < 1e-11
+
+
+@pytest.mark.parametrize("bw,F,prec", [(32, 1025, 2), (64, 257, 2), (200, 80, 2), (255, 65, 2), (512, 33, 2), (32, 600, 3),
+                                       (64, 257, 3), (512, 33, 3)])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_order_and_pair_workgroups_agree(env, bw, F, prec, fmt):
+    # Mixed and split calls of few GEMM workgroups run one order per workgroup,
+    # others order pairs: a field's results are the same bit for bit (255: an
+    # odd bandwidth's middle order; last column blocks partly filled).
+    S, torch, dev = env
+    n = 2 * bw
+    print(f"order workgroups bw={bw} F={F} prec={prec} fmt={fmt}", flush=True)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(bw)
+    g, h = (torch.randn((F, n, n), generator=gen, dtype=torch.float64, device=dev) for _ in range(2))
+    a, b = (torch.empty((F, bw * bw), dtype=torch.float64, device=dev) for _ in range(2))
+    x, y = torch.empty_like(g), torch.empty_like(g)
+    c, d = torch.empty_like(a[:3]), torch.empty_like(a[:3])
+    u, v = torch.empty_like(g[:3]), torch.empty_like(g[:3])
+    with contextlib.closing(S.Plan(bw, F, precision=prec)) as plan:
+        plan.forward(g, h, a, b, data_format=fmt)
+        plan.inverse(a, b, x, y, data_format=fmt)
+        plan.forward(g[:3], h[:3], c, d, data_format=fmt)
+        plan.inverse(c, d, u, v, data_format=fmt)
+        torch.cuda.synchronize()
+    assert torch.equal(c, a[:3]) and torch.equal(d, b[:3])
+    assert torch.equal(u, x[:3]) and torch.equal(v, y[:3])
