@@ -39,14 +39,18 @@ namespace s2 {
 // block-wide FFTs in LDS
 // ---------------------------------------------------------------------------
 
-// Division by a divisor 1 <= d < 2^16 of a value x < 2^16: floor(x/d) =
-// (x * ceil(2^32/d)) >> 32 (the rounding error x*(ceil(2^32/d)*d - 2^32)/2^32
-// stays below 1/d).
-__device__ __forceinline__ unsigned long long magic16(unsigned d) {
-    // ceil(2^32/d) = floor((2^32-1)/d) + 1 for d >= 2 (a 32-bit division)
-    return d == 1 ? 0x100000000ull : (unsigned long long)(0xFFFFFFFFu / d) + 1;
+// x / d for 0 <= x < 2^16 and a block-uniform 1 <= d < 2^16, exact: (x + 1/2) / d
+// is at least 1/(2d) from an integer, and the rounding errors (reciprocal r,
+// product) stay below x/d 2^-21.  Three full-rate instructions, where the 64-bit
+// product with ceil(2^32/d) took quarter-rate ones; r in a scalar register
+// (in a vector one the FP64 register passes took twice as long).
+// Ring FFT launches, us, forward / inverse: FP64 bw=255 x256 531 / 544 -> 530 / 525,
+// bw=300 x16 68 / 70 -> 63 / 62, FP32 bw=263 x64 374 / 378 -> 344 / 344, bw=37
+// x500 66 / 66 -> 61 / 61.
+__device__ __forceinline__ float magic16(int d) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, __builtin_amdgcn_rcpf((float)d))));
 }
-__device__ __forceinline__ int div16(int x, unsigned long long mg) { return (int)(((unsigned long long)x * mg) >> 32); }
+__device__ __forceinline__ int div16(int x, float r) { return (int)__builtin_fmaf((float)x, r, 0.5f * r); }
 
 // Threads of the mixed-radix and Bluestein instances (two blocks of 8 waves
 // per CU keep their LDS passes' latency covered).
@@ -164,7 +168,7 @@ __device__ __forceinline__ void mr_reg_pass(T* a, int N, int Ns, int nfft, const
     using F = typename Real<T>::type;
     constexpr int H = (R - 1) / 2;
     const int NR = N / R, step = N / (Ns * R);
-    const unsigned long long mNR = magic16(NR), mNs = magic16(Ns);
+    const float mNR = magic16(NR), mNs = magic16(Ns);
     const int total = nfft * NR;
     T v[PER][R];
 #pragma unroll
@@ -344,7 +348,7 @@ __device__ __forceinline__ void bluestein_rows(T* a, int N, int M, int nfft, con
     constexpr int V = rm_elems<T>() / kMrThreads;
     constexpr bool p2 = P2;  // is_pow2(M): separate instances keep each path's registers
     const int S = blu_stride(M), rows = blu_rows<T>(M), tot = rows * M;
-    const unsigned long long mM = magic16(M);
+    const float mM = magic16(M);
     const T* __restrict__ w = g + M;
     const T* __restrict__ bh = g + M + N;
     for (int i = threadIdx.x; i < tot; i += kMrThreads) {
@@ -379,7 +383,7 @@ __device__ __forceinline__ void bluestein_rows(T* a, int N, int M, int nfft, con
     } else {
         mr_reg_fft<T, -1, kBluMaxPrime>(a, M, rows, twl, RowsOf{M});
     }
-    const unsigned long long mN = magic16(N);
+    const float mN = magic16(N);
     for (int i = threadIdx.x; i < nfft * N; i += kMrThreads) {
         const int r = div16(i, mN), k = i - r * N;
         T c = w[k];
@@ -403,7 +407,7 @@ __device__ __forceinline__ int lds_rows(int rpb, int logN) {
 }
 // LDS position of the flat index i = row * N + column.
 template <int MODE>
-__device__ __forceinline__ int lds_row(int i, int N, int RS, unsigned long long mN) {
+__device__ __forceinline__ int lds_row(int i, int N, int RS, float mN) {
     if constexpr (MODE >= 2) {
         const int r = div16(i, mN);
         return r * RS + (i - r * N);
@@ -475,7 +479,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     const int nr = min(rpb, N - j0);
     const size_t base = ((size_t)f * N + j0) * N;
     const int tot = nr * N;  // < 2^16 (div16)
-    const unsigned long long mN = magic16(N);
+    const float mN = magic16(N);
     using F = typename Real<T>::type;
     for (int i0 = threadIdx.x; i0 < tot; i0 += FB * blockDim.x) {
         double vr[FB], vi[FB];
@@ -497,7 +501,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     if constexpr (MODE != 0) twp = stage_fft_twiddles<T, MODE>(b, N, logN, tw);
     __syncthreads();
     T* r = fft_rows<T, -1, MODE>(a, b, N, logN, pow2, nr, twp, tw);
-    const unsigned long long mnr = magic16(nr);
+    const float mnr = magic16(nr);
     const int out = real ? tot >> 1 : tot;  // REAL data: rows below bw (see k_fphi_fwd)
     for (int i = threadIdx.x; i < out; i += blockDim.x) {
         const int row = div16(i, mnr), jl = i - row * nr;
@@ -523,7 +527,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     const int q0 = bx * rpb;
     const int nr = min(rpb, nrows - q0);
     const int tot = nr * N;  // < 2^16 (div16)
-    const unsigned long long mN = magic16(N);
+    const float mN = magic16(N);
     for (int i0 = threadIdx.x; i0 < tot; i0 += FB * blockDim.x) {
         T xv[FB];
         double wv[FB];
@@ -552,7 +556,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     if constexpr (MODE != 0) twp = stage_fft_twiddles<T, MODE>(b, N, logN, tw);
     __syncthreads();
     T* V = fft_rows<T, -1, MODE>(a, b, N, logN, pow2, nr, twp, tw);
-    const unsigned long long mB = magic16(B);
+    const float mB = magic16(B);
     for (int i = threadIdx.x; i < nr * B; i += blockDim.x) {
         const int rl = div16(i, mB), k = i - rl * B;
         const int r = row_of(q0 + rl, N, cut);
@@ -1154,7 +1158,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     // V[k] = e^{+i pi k/2N} (X[k] - i X[N-k]), X[N] = 0, X[k >= B] = 0: one
     // of the two terms is nonzero, X[k] for k < B, X[N-k] for k > B.
     const int tot = nr * N;  // < 2^16 (div16)
-    const unsigned long long mN = magic16(N);
+    const float mN = magic16(N);
     for (int i0 = threadIdx.x; i0 < tot; i0 += FB * blockDim.x) {
         T xv[FB], e[FB];
 #pragma unroll
@@ -1260,7 +1264,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     const int j0 = bx * rpb;
     const int nr = min(rpb, N - j0);
     const int tot = nr * N;  // < 2^16 (div16)
-    const unsigned long long mnr = magic16(nr);
+    const float mnr = magic16(nr);
     const int in = real ? tot >> 1 : tot;
     for (int i0 = threadIdx.x; i0 < in; i0 += FB * blockDim.x) {
         T v[FB];
@@ -1287,7 +1291,7 @@ __global__ __launch_bounds__(MODE ? kMrThreads : 256) S2_FFT_OCCUPANCY(MODE) voi
     __syncthreads();
     T* y = fft_rows<T, +1, MODE>(a, b, N, logN, pow2, nr, twp, tw);
     const size_t base = ((size_t)f * N + j0) * N;
-    const unsigned long long mN = magic16(N);
+    const float mN = magic16(N);
     for (int i = threadIdx.x; i < tot; i += blockDim.x) {
         const T v = y[lds_row<MODE>(i, N, RS, mN)];
         re[base + i] = (double)v.x;

@@ -46,14 +46,11 @@ constexpr int kPrimeMaxN = 1024;  // ring lengths up to it hold one prime factor
 
 typedef double pvec4 __attribute__((ext_vector_type(4)));
 
-// x / d for 0 <= x < 2^16, exact: (x + 1/2) / d is at least 1/(2d) from an
-// integer, and the product's rounding errors (r within 2^-22) stay below
-// x/d 2^-21.  Three full-rate instructions; the 32-bit products of div16 run
-// at a quarter of the rate.
+// div16 with its divisor and remainder (the reciprocals are per block)
 struct DivF {
     int d;
     float r;  // 1/d
-    __device__ __forceinline__ int quo(int x) const { return (int)__builtin_fmaf((float)x, r, 0.5f * r); }
+    __device__ __forceinline__ int quo(int x) const { return div16(x, r); }
     __device__ __forceinline__ int rem(int x, int q) const { return x - __mul24(q, d); }
     __device__ __forceinline__ int rem(int x) const { return rem(x, quo(x)); }
 };
@@ -204,7 +201,7 @@ __device__ __forceinline__ void prime_parts(double2* a, int nr, const PrimeDft& 
     double2* twl = a + d.P * rs;
     for (int i = threadIdx.x; i < R; i += kMrThreads) twl[i] = tw[4 + i];
     __syncthreads();
-    const unsigned long long mnr = magic16(nr);
+    const float mnr = magic16(nr);
     mr_reg_fft<double2, SIGN>(a, R, d.P * nr, twl, [=](int f) { return f * R + div16(f, mnr); });
     const DivF dc = div_by(nc);
     for (int i = threadIdx.x; i < d.H * nc; i += kMrThreads) {
