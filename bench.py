@@ -22,7 +22,7 @@ Also reported on the same JSON line:
               same fields, with their errors against FP64; and the FP64 form
               at cutoff = bw/4 (naive branch for orders >= 64);
   non_pow2    FP64 and mixed pairs/s at bw=255 (register mixed-radix FFTs)
-              beside bw=256, bw=127 and bw=263 (Bluestein FFTs) beside bw=128,
+              beside bw=256, bw=127 and bw=263 (one large prime) beside bw=128,
               256 fields, and the bw=255 / 127 batches against their per-field path;
   cpu_baseline  the CPU FP64 oracle (a port of the reference path) timed on
               the host, one process per core, on a bounded sample.
@@ -205,9 +205,9 @@ MFMA_PEAK = {"fp64": (78.6, 1), "fp32": (157.3, 1), "mixed": (157.3, 1), "split"
 def non_pow2(dev, steps):
     """FP64 plans at bandwidths whose grids are not powers of two, beside the
     power of two next to them, 256 fields each: bw=255 (510 = 2*3*5*17 rings:
-    register mixed-radix FFTs and DCTs), bw=127 (254 = 2*127: Bluestein, a
-    convolution of length 512) and bw=263 (526 = 2*263: Bluestein, length
-    1080 = 2^3 3^3 5); MFMA Legendre GEMMs throughout.  The bw=255 and bw=127
+    register mixed-radix FFTs), bw=127 (254 = 2*127) and bw=263 (526 = 2*263),
+    FP64 on prime-factor DFTs, FP32 on Bluestein FFTs (convolution lengths 512
+    and 1080 = 2^3 3^3 5); MFMA Legendre GEMMs throughout.  The bw=255 and bw=127
     batches are checked against the drop-ins (per-field kernels) on their
     first field.  The mixed form (FP32 ring FFTs, naive GEMMs over rings
     padded to whole 64-ring groups) is timed on the same fields, with its
