@@ -694,3 +694,35 @@ def test_order_and_pair_workgroups_agree(env, bw, F, prec, fmt):
         torch.cuda.synchronize()
     assert torch.equal(c, a[:3]) and torch.equal(d, b[:3])
     assert torch.equal(u, x[:3]) and torch.equal(v, y[:3])
+
+
+@pytest.mark.parametrize("bws", [(24,), (24, 40), (16, 24, 33, 46, 64, 90, 128)])
+@pytest.mark.parametrize("prec", [0, 2])
+def test_conv_batch_branches(env, bws, prec):
+    # A batch's groups run as branches of one graph (one group, one group per
+    # branch, several groups on a branch): every replay, with eager work between
+    # the replays, equals the plans' own convolutions bit for bit.
+    S, torch, dev = env
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(sum(bws))
+    reqs, grids = [], {}
+    for bw in bws:
+        n, F = 2 * bw, 2 + bw % 3
+        grids[bw] = [torch.randn((F, n, n), generator=gen, dtype=torch.float64, device=dev) for _ in range(4)]
+        grids[bw] += [torch.empty_like(grids[bw][0]) for _ in range(2)]
+        reqs += [(bw, *[t[f] for t in grids[bw]]) for f in range(F)]
+    batch = S.ConvBatch(reqs[::2] + reqs[1::2], precision=prec)
+    for _ in range(3):
+        for bw in bws:
+            grids[bw][4].zero_()
+            grids[bw][5].zero_()
+        batch.run()
+        torch.cuda.synchronize()
+        for bw in bws:
+            g = grids[bw]
+            a, b = torch.empty_like(g[0]), torch.empty_like(g[0])
+            p = prec if prec == 0 or bw >= 32 else 0
+            with contextlib.closing(S.Plan(bw, g[0].shape[0], precision=p)) as plan:
+                plan.conv(*g[:4], a, b)
+                torch.cuda.synchronize()
+            assert torch.equal(a, g[4]) and torch.equal(b, g[5])
