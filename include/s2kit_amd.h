@@ -126,7 +126,10 @@ int s2amd_conv(s2amd_plan* plan, const double* sre, const double* sim, const dou
  * gathering each group's grids into contiguous staging buffers (skipped for
  * an array whose requests already lie back to back in request order), the
  * group's forward / zonal / TransMult / inverse pipeline, scattering the
- * outputs -- as one HIP graph; _run replays it on a stream.  Requests are
+ * outputs -- as one HIP graph; _run replays it on a stream.  Groups whose
+ * memory is disjoint run beside each other; if an output grid of one group
+ * overlaps a grid of another, the groups run one after another in ascending
+ * bandwidth.  Requests are
  * copied at creation: their buffers must stay allocated while the batch is
  * used; their contents are read at every _run.  precision: S2AMD_FP64,
  * S2AMD_MIXED or S2AMD_SPLIT_BF16; a group whose bandwidth the chosen form does

@@ -7,8 +7,8 @@
 // already back to back in request order are gathered into contiguous staging
 // buffers first, and outputs scattered back, by the copy kernels below.  The
 // whole batch is recorded once as a HIP graph on library streams, its groups on
-// parallel branches, and replayed by s2amd_conv_batch_run, so a repeated batch
-// costs one launch.
+// parallel branches unless their grids overlap, and replayed by
+// s2amd_conv_batch_run, so a repeated batch costs one launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "s2_internal.h"
+#include "s2_overlap.h"
 
 extern "C" {
 #include "s2kit_amd.h"
@@ -60,10 +61,7 @@ struct ConvGroup {
 
 // Streams and events a batch's branches are captured with (branch 0 on the
 // batch's own stream); the graph needs none of them afterwards.
-#ifndef S2_BATCH_BRANCHES
-#define S2_BATCH_BRANCHES 3
-#endif
-constexpr size_t kBranches = S2_BATCH_BRANCHES;  // 1 / 2 / 3 / 4 / 5: 1230 / 1074 / 1023 / 1048 / 1102 us for the batch below
+constexpr size_t kBranches = 3;  // 1 / 2 / 3 / 4 / 5: 1230 / 1074 / 1023 / 1048 / 1102 us for the batch below
 struct Branches {
     hipEvent_t fork = nullptr;
     std::vector<hipStream_t> stream;
@@ -222,17 +220,30 @@ extern "C" int s2amd_conv_batch_create(s2amd_conv_batch** out, const s2amd_conv_
                 S2_HIP(hipMemcpy(g.scatter_dst, sdst.data(), sizeof(void*) * sdst.size(), hipMemcpyHostToDevice));
             }
         }
-        // record the batch: the groups share nothing (plans, staging and grids of
-        // their own), so they run on up to kBranches branches of the graph between
+        // record the batch: the groups have plans and staging of their own, so
+        // they run on up to kBranches branches of the graph between
         // one fork and one join, the largest first, each group on the branch with
         // the least so far; small groups' launches then fill the chip beside the
         // large ones' (512 requests of
-        // bw 32 to 512, mixed, 1230 -> 1023 us; 64 in FP64 409 us on four branches, 393 on three)
+        // bw 32 to 512, mixed, 1230 -> 1023 us; 64 in FP64 409 us on four branches, 393 on three).
+        // The grids are the caller's: where a group writes memory that another
+        // reads or writes, all run on one branch in ascending bandwidth
         const auto size = [](const ConvGroup* g) { return (long)g->bw * g->bw * g->n; };
         std::vector<ConvGroup*> order;
         for (ConvGroup& g : b->groups) order.push_back(&g);
-        std::sort(order.begin(), order.end(), [&](const ConvGroup* x, const ConvGroup* y) { return size(x) > size(y); });
-        Branches br(b->stream, std::min<size_t>(kBranches, order.size()));
+        std::vector<MemRange> grids;
+        for (int i = 0; i < n; ++i) {
+            const s2amd_conv_request& r = req[i];
+            const size_t bytes = sizeof(double) * 4 * r.bw * r.bw;
+            for (const double* q : {r.sre, r.sim, r.hre, r.him})
+                grids.push_back({(uintptr_t)q, (uintptr_t)q + bytes, r.bw, false});
+            for (const double* q : {r.ore, r.oim}) grids.push_back({(uintptr_t)q, (uintptr_t)q + bytes, r.bw, true});
+        }
+        const bool ordered = groups_conflict(std::move(grids));
+        if (!ordered)
+            std::sort(order.begin(), order.end(),
+                      [&](const ConvGroup* x, const ConvGroup* y) { return size(x) > size(y); });
+        Branches br(b->stream, ordered ? 1 : std::min<size_t>(kBranches, order.size()));
         std::vector<long> load(br.stream.size(), 0);
         S2_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
         try {
