@@ -84,7 +84,7 @@ KERNELS = {
 
 
 def dense_fp64(form, bw, nfields):
-    """The FP64 call runs the dense Legendre GEMMs (s2_naive64.hip) and no DCT stage."""
+    """Calls of an FP64 plan of nfields fields run the dense Legendre GEMMs (s2_naive64.hip) and no DCT stage."""
     return form == "fp64" and 16 <= bw <= 512 and (bw <= 320 or nfields >= 4)
 
 

@@ -32,10 +32,11 @@ enum {
 
 /* Arithmetic of the transforms (inputs and outputs are FP64 in every form). */
 typedef enum {
-    /* FP64 throughout, on FP64 MFMA: at bw <= 320, and up to 512 for calls of
-     * four fields or more, every order as a dense sum over the rings
-     * (naive.c's form), else seminaive (DCT + cosine-series tables).  The same
-     * transform to rounding; matches the reference to ~1e-13. */
+    /* FP64 throughout, on FP64 MFMA: plans at bw <= 320, and up to 512 with
+     * max_fields >= 4, take every order as a dense sum over the rings
+     * (naive.c's form), others seminaive (DCT + cosine-series tables).  The same
+     * transform to rounding (~1e-13, also between two plans at bw 321 .. 512 of
+     * which one has max_fields < 4); matches the reference to ~1e-13. */
     S2AMD_FP64 = 0,
     /* seminaive in FP32 (FFTs, DCTs, FP32-MFMA projections). Measured error
      * 1e-6 .. 4e-5 relative: the cosine-space sums cancel.  bw a power of two
@@ -57,9 +58,11 @@ typedef struct s2amd_plan s2amd_plan;
 
 /* Plan for bandwidth bw (2..1024), up to max_fields fields per call,
  * seminaive for orders < cutoff and naive (naive.c) for orders >= cutoff
- * (cutoff = bw: all seminaive; where an FP64 call runs the dense sums, the
+ * (cutoff = bw: all seminaive; where an FP64 plan runs the dense sums, the
  * cutoff decides which orders of an odd bw keep the seminaive synthesis of
- * degree bw-1).  Generates the forward and transposed tables
+ * degree bw-1).  A field's results do not depend on the field count of its call,
+ * bit for bit, except that single fields of FP64 plans on the seminaive sums at
+ * bw >= 512 run a GEMV of their own order of sums.  Generates the forward and transposed tables
  * on the current device.  FP64 plans with bw in [16, 1024] and FP32 plans on
  * power-of-two grids with bw in [32, 1024] run both branches as MFMA GEMMs at
  * any cutoff (FP64 grids that are not powers of two on mixed-radix FFTs);

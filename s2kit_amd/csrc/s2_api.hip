@@ -350,25 +350,22 @@ struct Plan {
     DevConsts c;
     DevTables t;
     GemmTables g;
-    GemmTables gd;  // FP64, bw <= 512: dense tables (s2_naive64.hip), for calls of dense_min fields or more
-    int dense_min = 0;  // 0: none
     DBuf X, Cb, cr, ci, zr, zi;
     StageTimer timer;
 };
 
-// FP64 plans: the GEMM path from two fields per call, and for one field below
-// bw = 512; single fields at bw >= 512 go to the per-field kernels, whose row
-// GEMVs stream the tables faster than one field's GEMM tiles use them
-// (measured on MI355X, us per fwd+inv call, GEMM vs per-field: bw=256 F=1
-// 75 vs 88; bw=512 F=1 210 vs 205, F=2 266 vs 336; bw=1024 F=1 1389 vs 1239).
+// FP64 plans without the dense tables: the GEMM path from two fields per call,
+// and for one field below bw = 512; single fields at bw >= 512 go to the
+// per-field kernels, whose row GEMVs stream the tables faster than one field's
+// seminaive GEMM tiles use them (measured on MI355X, us per fwd+inv call, GEMM
+// vs per-field: bw=512 F=1 210 vs 205, F=2 266 vs 336; bw=1024 F=1 1389 vs 1239).
+// Plans with the dense tables run every call on them: a field's results then do
+// not depend on the field count of its call.
 static bool use_fast(const Plan* p, int F) {
     if (!p->fast) return false;
-    if (p->precision != S2AMD_FP64) return true;
+    if (p->precision != S2AMD_FP64 || p->g.n64) return true;
     return F >= 2 || p->bw < 512;
 }
-
-// The GEMM tables of a call of F fields.
-static GemmTables& gemm_of(Plan* p, int F) { return p->dense_min && F >= p->dense_min ? p->gd : p->g; }
 
 // The forward pipeline of a plan on scratch X (order-major intermediate) and
 // Cb (cosine rows; unused by the mixed and split-BF16 forms).
@@ -377,7 +374,7 @@ static void plan_forward_on(Plan* p, const double* re, const double* im, double*
     if (p->precision == S2AMD_MIXED || p->precision == S2AMD_SPLIT_BF16)
         forward_mixed(p->c, p->g, re, im, cre, cim, F, fmt, X, s, tm);
     else if (use_fast(p, F))
-        forward_fast(p->c, gemm_of(p, F), re, im, cre, cim, F, fmt, X, Cb, s, tm);
+        forward_fast(p->c, p->g, re, im, cre, cim, F, fmt, X, Cb, s, tm);
     else
         forward_fp64(p->c, p->t, re, im, cre, cim, F, fmt, (double2*)X, (double2*)Cb, s, tm);
 }
@@ -432,7 +429,7 @@ static void plan_inverse(Plan* p, const double* cre, const double* cim, double* 
     if (p->precision == S2AMD_MIXED || p->precision == S2AMD_SPLIT_BF16)
         inverse_mixed(p->c, p->g, cre, cim, re, im, F, fmt, p->X.p, s, &p->timer);
     else if (use_fast(p, F))
-        inverse_fast(p->c, gemm_of(p, F), cre, cim, re, im, F, fmt, p->X.p, p->Cb.p, s, &p->timer);
+        inverse_fast(p->c, p->g, cre, cim, re, im, F, fmt, p->X.p, p->Cb.p, s, &p->timer);
     else
         inverse_fp64(p->c, p->t, cre, cim, re, im, F, fmt, p->X.as<double2>(), p->Cb.as<double2>(), s, &p->timer);
 }
@@ -1079,14 +1076,10 @@ extern "C" int s2amd_plan_create(s2amd_plan** out, int bw, int cutoff, int max_f
                 p->fast = fast_supported(bw, cutoff, precision);
                 // one field at bw >= 512 runs on the per-field kernels (use_fast)
                 const bool one = precision == S2AMD_FP64 && max_fields == 1 && bw >= 512;
-                if (p->fast && !one) {
-                    const int least = n64_min_fields(bw);
-                    if (n64_supported(bw, precision) && max_fields >= least) {
-                        p->dense_min = least;
-                        n64_tables_create(p->gd, p->t, p->c, s);
-                    }
-                    if (p->dense_min != 1) gemm_tables_create(p->g, p->t, precision, s);
-                }
+                if (p->fast && n64_supported(bw, precision) && max_fields >= n64_min_fields(bw))
+                    n64_tables_create(p->g, p->t, p->c, s);
+                else if (p->fast && !one)
+                    gemm_tables_create(p->g, p->t, precision, s);
             }
             const size_t N = 2 * (size_t)bw, F = max_fields;
             // large enough for the fast layouts and for the FP64 zonal transform
@@ -1102,7 +1095,6 @@ extern "C" int s2amd_plan_create(s2amd_plan** out, int bw, int cutoff, int max_f
             consts_destroy(p->c);
             tables_destroy(p->t);
             gemm_tables_destroy(p->g);
-            gemm_tables_destroy(p->gd);
             for (DBuf* b : {&p->X, &p->Cb, &p->cr, &p->ci, &p->zr, &p->zi}) b->release();
             throw;
         }
@@ -1143,7 +1135,7 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
         const bool mixed = p->precision == S2AMD_MIXED;
         if (!gemm && !mixed) return;  // nothing to choose for this plan and field count
         const size_t N = 2 * (size_t)p->bw, F = nfields;
-        GemmTables& g = gemm_of(p, nfields);
+        GemmTables& g = p->g;
         struct Scratch {  // temporary fields, freed on every exit
             DBuf re, im, cr, ci;
             ~Scratch() {
@@ -1194,9 +1186,8 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
 extern "C" int s2amd_plan_tuning(const s2amd_plan* p, int* cols, int* col_tiles, int* ring_groups) {
     return run_plan("s2amd_plan_tuning", [&] {
         if (!p) throw ArgError{"plan is NULL"};
-        const GemmTables& g = p->dense_min && p->gd.t_ncb ? p->gd : p->g;
-        if (cols) *cols = g.t_ncb;
-        if (col_tiles) *col_tiles = g.t_ct;
+        if (cols) *cols = p->g.t_ncb;
+        if (col_tiles) *col_tiles = p->g.t_ct;
         if (ring_groups) *ring_groups = p->g.t_gj;
     });
 }
@@ -1210,7 +1201,6 @@ extern "C" int s2amd_plan_destroy(s2amd_plan* p) {
         consts_destroy(p->c);
         tables_destroy(p->t);
         gemm_tables_destroy(p->g);
-        gemm_tables_destroy(p->gd);
         for (DBuf* b : {&p->X, &p->Cb, &p->cr, &p->ci, &p->zr, &p->zi}) b->release();
         delete p;
     });
@@ -1221,8 +1211,8 @@ extern "C" size_t s2amd_plan_bytes(const s2amd_plan* p) {
     const size_t el = p->precision == S2AMD_FP64        ? sizeof(double)
                       : p->precision == S2AMD_SPLIT_BF16 ? sizeof(uint16_t)
                                                          : sizeof(float);  // GEMM table elements
-    return 2 * sizeof(double) * p->t.total + el * (p->g.nf + p->g.ni) + sizeof(double) * (p->gd.nf + p->gd.ni) + p->X.n + p->Cb.n + p->cr.n + p->ci.n +
-           p->zr.n + p->zi.n;
+    return 2 * sizeof(double) * p->t.total + el * (p->g.nf + p->g.ni) + p->X.n + p->Cb.n + p->cr.n + p->ci.n + p->zr.n +
+           p->zi.n;
 }
 
 extern "C" int s2amd_plan_tables(const s2amd_plan* p, const double** fwd, const double** inv, long* n) {

@@ -1,5 +1,5 @@
 // Batched GEMM path, FP64 or FP32 arithmetic (FP64 inputs and outputs either
-// way).  FP64 calls at bw <= 512 (from four fields above bw = 320) run the
+// way).  FP64 plans at bw <= 512 (of four fields or more above bw = 320) run the
 // dense GEMMs of s2_naive64.hip instead of the DCT and GEMM stages below,
 // around the same ring FFTs.  Power-of-two grids (N = 2*bw = 64 .. 2048):
 //

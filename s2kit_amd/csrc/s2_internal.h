@@ -235,7 +235,7 @@ void gemm_tables_create(GemmTables& g, const DevTables& t, int prec, hipStream_t
 void gemm_tables_destroy(GemmTables& g);
 // ---- dense FP64 Legendre GEMMs (s2_naive64.hip) ---------------------------
 bool n64_supported(int bw, int prec);  // FP64, bw in [16, 512]
-int n64_min_fields(int bw);            // fields per call from which they beat the seminaive tables
+int n64_min_fields(int bw);            // largest call of a plan from which it holds them
 void n64_tables_create(GemmTables& g, const DevTables& t, const DevConsts& c, hipStream_t s);
 void n64_fwd_launch(const DevConsts& c, const GemmTables& g, const double2* X, double* cre, double* cim, int F, Fmt fmt,
                     hipStream_t s);

@@ -116,13 +116,16 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void k
 // as the seminaive tables' 1.4 GB.
 bool n64_supported(int bw, int prec) { return prec == 0 && bw >= 16 && bw <= 512; }
 
-// Fields per call from which the dense tables beat the seminaive ones (DCT
-// included): always up to bw = 320; above, one to three fields are bound by
-// the table stream, three times as long here (us per forward / inverse,
-// dense against seminaive: bw=300 x1 35 / 24 against 38 / 36, bw=400 x2
+// Fields per call (the plan's largest) from which the dense tables beat the
+// seminaive ones (DCT included): always up to bw = 320; above, one to three
+// fields are bound by the table stream, three times as long here (us per forward
+// / inverse, dense against seminaive: bw=300 x1 35 / 24 against 38 / 36, bw=400 x2
 // 77 / 69 against 63 / 64, x4 82 / 75 against 87 / 88, bw=512 x2 143 / 110
 // against 104 / 98, x4 152 / 118 against 144 / 128, x8 173 / 131 against
-// 217 / 210).
+// 217 / 210).  A plan holds one kind and runs its smaller calls on it as well
+// (one field, dense against seminaive: bw=400 85 / 65 against 58 / 57, bw=512
+// 147 / 124 against 72 / 80): with both, a field's last bits depended on its
+// call's field count, and a plan held two table sets (bw=512 x8 2201 -> 1670 MB).
 int n64_min_fields(int bw) { return bw <= 320 ? 1 : 4; }
 
 void n64_tables_create(GemmTables& g, const DevTables& t, const DevConsts& c, hipStream_t s) {
@@ -199,7 +202,11 @@ static void n64_inv_direct(const DevConsts& c, const GemmTables& g, const double
 
 void n64_fwd_launch(const DevConsts& c, const GemmTables& g, const double2* X, double* cre, double* cim, int F, Fmt fmt,
                     hipStream_t s) {
-    const int B = c.bw, kc = n64_kc_cols(B, F);
+    // bw > 384: the forward table exceeds the 256 MB memory-side cache, and the
+    // direct kernel's waves keep too little of the HBM stream in flight (one field,
+    // us, direct / 32 columns: bw=360 55 / 71, bw=400 129 / 85, bw=512 206 / 147;
+    // the inverse stays direct, bw=400 65 / 92, bw=512 124 / 120)
+    const int B = c.bw, kc = n64_kc_cols(B, F) ? n64_kc_cols(B, F) : B > 384 ? 32 : 0;
     if (kc == 64) return (B <= 256 ? n64_fwd_kc_launch<1, 4> : n64_fwd_kc_launch<2, 4>)(c, g, X, cre, cim, F, fmt, s);
     if (kc == 32) return (B <= 256 ? n64_fwd_kc_launch<1, 2> : n64_fwd_kc_launch<2, 2>)(c, g, X, cre, cim, F, fmt, s);
     // tiles per wave: more reuse each load more, fewer give more waves and a

@@ -1,0 +1,66 @@
+"""Which kernels a plan's calls run changes no result of the plan."""
+import contextlib
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    import s2kit_amd
+    s2kit_amd.lib()
+    return s2kit_amd, torch, torch.device("cuda:0")
+
+
+def grids(torch, dev, bw, F, seed, planes=2):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    return [torch.randn((F, 2 * bw, 2 * bw), generator=gen, dtype=torch.float64, device=dev) for _ in range(planes)]
+
+
+def pair(torch, plan, g, h, fmt):
+    """Coefficients of the grids, and the grids of those coefficients."""
+    F, n = g.shape[:2]
+    a, b = (torch.empty((F, n * n // 4), dtype=torch.float64, device=g.device) for _ in range(2))
+    x, y = torch.empty_like(g), torch.empty_like(g)
+    plan.forward(g, h, a, b, data_format=fmt)
+    plan.inverse(a, b, x, y, data_format=fmt)
+    return a, b, x, y
+
+
+@pytest.mark.parametrize("bw,F", [(257, 4), (257, 5), (257, 16), (300, 4), (320, 17), (321, 5), (321, 16), (400, 17),
+                                  (511, 4), (512, 5)])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_results_do_not_depend_on_the_field_count(env, bw, F, fmt):
+    # FP64 plans from bw = 257 to 512, at the field counts where calls change
+    # kernels: the fields of a call have the same bits in calls of one, two and
+    # three fields on the same plan, and after it was autotuned.
+    S, torch, dev = env
+    print(f"field counts bw={bw} F={F} fmt={fmt}", flush=True)
+    g, h = grids(torch, dev, bw, F, bw + F)
+    with contextlib.closing(S.Plan(bw, F)) as plan:
+        whole = pair(torch, plan, g, h, fmt)
+        for k in (1, 2, 3):
+            for u, v in zip(pair(torch, plan, g[:k], h[:k], fmt), whole):
+                assert torch.equal(u, v[:k]), k
+        plan.autotune(F)
+        for k in (F, 1):
+            for u, v in zip(pair(torch, plan, g[:k], h[:k], fmt), whole):
+                assert torch.equal(u, v[:k]), k
+
+
+@pytest.mark.parametrize("bw", [321, 512])
+def test_convolutions_do_not_depend_on_the_field_count(env, bw):
+    S, torch, dev = env
+    F = 5
+    print(f"conv field counts bw={bw}", flush=True)
+    t = grids(torch, dev, bw, F, bw, 4)
+    a, b, x, y = (torch.empty_like(t[0]) for _ in range(4))
+    with contextlib.closing(S.Plan(bw, F)) as plan:
+        plan.conv(*t, a, b)
+        for f in range(F):
+            plan.conv(*[v[f:f + 1] for v in t], x[f:f + 1], y[f:f + 1])
+    assert torch.equal(a, x) and torch.equal(b, y)
