@@ -74,12 +74,16 @@ int s2amd_plan_destroy(s2amd_plan* plan);
 /* Autotuning (no counterpart in the reference): times forward+inverse of
  * nfields fields on stream for each tile shape the plan's GEMMs accept
  * (FP64/FP32: data columns per block and column tiles per table load; mixed:
- * 64-ring groups per inverse block) and keeps the fastest for later calls.
+ * 64-ring groups per inverse block) and keeps the fastest for later calls; on
+ * the dense FP64 sums, where a call's data columns decide its kernels, for calls
+ * of as many columns (four per COMPLEX field, two per REAL one), and the K-chunked
+ * kernels of larger calls have one shape only.  COMPLEX calls are timed.
  * Every shape computes the same sums in the same order: results do not
  * change.  Allocates and frees temporary device fields; synchronises the
  * stream.  Plans whose calls of nfields fields take no GEMM (or split-BF16
  * plans) keep their defaults.  s2amd_plan_tuning reports the choice (0: the
- * built-in heuristic). */
+ * built-in heuristic; dense FP64: columns per inverse block or wave, column tiles
+ * per forward wave). */
 int s2amd_plan_autotune(s2amd_plan* plan, int nfields, void* stream);
 int s2amd_plan_tuning(const s2amd_plan* plan, int* cols, int* col_tiles, int* ring_groups);
 /* Device bytes held by the plan (tables + scratch). */
@@ -150,8 +154,8 @@ typedef struct {
 } s2amd_conv_request;
 
 typedef struct s2amd_conv_batch s2amd_conv_batch;
-/* Groups the requests by bandwidth, creates and autotunes (s2amd_plan_autotune)
- * one plan per group, and records the whole batch as one HIP graph. */
+/* Groups the requests by bandwidth, creates and autotunes (s2amd_plan_autotune,
+ * on REAL calls) one plan per group, and records the whole batch as one HIP graph. */
 int s2amd_conv_batch_create(s2amd_conv_batch** batch, const s2amd_conv_request* req, int n, int precision,
                             void* stream);
 int s2amd_conv_batch_run(s2amd_conv_batch* batch, void* stream);

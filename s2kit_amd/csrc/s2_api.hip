@@ -1105,15 +1105,15 @@ extern "C" int s2amd_plan_create(s2amd_plan** out, int bw, int cutoff, int max_f
 
 // Time plan_forward + plan_inverse of nfields zero fields on stream s:
 // best of two runs after a warm-up, in ms.
-static float time_pair(Plan* p, int F, hipStream_t s, double* re, double* im, double* cr, double* ci) {
+static float time_pair(Plan* p, int F, Fmt fmt, hipStream_t s, double* re, double* im, double* cr, double* ci) {
     hipEvent_t e0, e1;
     S2_HIP(hipEventCreate(&e0));
     S2_HIP(hipEventCreate(&e1));
     float best = 1e30f;
     for (int r = 0; r < 3; ++r) {
         S2_HIP(hipEventRecord(e0, s));
-        plan_forward(p, re, im, cr, ci, F, Fmt::Complex, s);
-        plan_inverse(p, cr, ci, re, im, F, Fmt::Complex, s);
+        plan_forward(p, re, im, cr, ci, F, fmt, s);
+        plan_inverse(p, cr, ci, re, im, F, fmt, s);
         S2_HIP(hipEventRecord(e1, s));
         S2_HIP(hipEventSynchronize(e1));
         float ms = 0;
@@ -1125,12 +1125,11 @@ static float time_pair(Plan* p, int F, hipStream_t s, double* re, double* im, do
     return best;
 }
 
-extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
+int s2::plan_autotune(s2amd_plan* p, int nfields, Fmt fmt, hipStream_t s) {
     return run_plan("s2amd_plan_autotune", [&] {
         if (!p) throw ArgError{"plan is NULL"};
         if (nfields < 1 || nfields > p->max_fields) throw ArgError{"nfields must be in [1, max_fields]"};
         DeviceGuard dg(p->device);
-        const hipStream_t s = (hipStream_t)stream;
         const bool gemm = (p->precision == S2AMD_FP64 || p->precision == S2AMD_FP32) && use_fast(p, nfields);
         const bool mixed = p->precision == S2AMD_MIXED;
         if (!gemm && !mixed) return;  // nothing to choose for this plan and field count
@@ -1144,24 +1143,34 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
         } t;
         struct Restore {  // the previous choice stays if a trial fails
             GemmTables& g;
-            int ncb, ct, gj;
+            int ncb, ct, cols, gj;
             bool done = false;
             ~Restore() {
-                if (!done) g.t_ncb = ncb, g.t_ct = ct, g.t_gj = gj;
+                if (!done) g.t_ncb = ncb, g.t_ct = ct, g.t_cols = cols, g.t_gj = gj;
             }
-        } keep{g, g.t_ncb, g.t_ct, g.t_gj};
+        } keep{g, g.t_ncb, g.t_ct, g.t_cols, g.t_gj};
+        const std::vector<std::pair<int, int>> tiles =
+            gemm ? gemm_tile_choices(g, nfields, fmt) : std::vector<std::pair<int, int>>{};
+        if (tiles.size() == 1) {  // nothing to time
+            g.t_ncb = tiles[0].first;
+            g.t_ct = tiles[0].second;
+            g.t_cols = 0;
+            keep.done = true;
+            return;
+        }
+        if (g.n64) g.t_cols = n64_cols(nfields, fmt);
         t.re.reserve(sizeof(double) * N * N * F);
         t.im.reserve(sizeof(double) * N * N * F);
         t.cr.reserve(sizeof(double) * p->bw * p->bw * F);
         t.ci.reserve(sizeof(double) * p->bw * p->bw * F);
         for (DBuf* b : {&t.re, &t.im, &t.cr, &t.ci}) S2_HIP(hipMemsetAsync(b->p, 0, b->n, s));
         auto run = [&] {
-            return time_pair(p, nfields, s, t.re.as<double>(), t.im.as<double>(), t.cr.as<double>(), t.ci.as<double>());
+            return time_pair(p, nfields, fmt, s, t.re.as<double>(), t.im.as<double>(), t.cr.as<double>(), t.ci.as<double>());
         };
         float best = 1e30f;
         if (gemm) {
             int bn = 0, bc = 0;
-            for (const auto& tc : gemm_tile_choices(g)) {
+            for (const auto& tc : tiles) {
                 g.t_ncb = tc.first;
                 g.t_ct = tc.second;
                 const float ms = run();
@@ -1181,6 +1190,10 @@ extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
         S2_HIP(hipStreamSynchronize(s));
         keep.done = true;
     });
+}
+
+extern "C" int s2amd_plan_autotune(s2amd_plan* p, int nfields, void* stream) {
+    return plan_autotune(p, nfields, Fmt::Complex, (hipStream_t)stream);
 }
 
 extern "C" int s2amd_plan_tuning(const s2amd_plan* p, int* cols, int* col_tiles, int* ring_groups) {

@@ -923,8 +923,8 @@ static void inv_launch(const DevConsts& c, const GemmTables& g, const double* cr
                (const GemmMeta*)g.meta, (R*)Cb, (T*)X, B, g.cut, mlo, F, ncb, (int)fmt);
 }
 
-std::vector<std::pair<int, int>> gemm_tile_choices(const GemmTables& g) {
-    if (g.n64) return {{16, 1}, {32, 2}};  // column tiles per wave
+std::vector<std::pair<int, int>> gemm_tile_choices(const GemmTables& g, int F, Fmt fmt) {
+    if (g.n64) return n64_tile_choices(g, F, fmt);
     const int bw = g.bw, prec = g.prec;
     const int row = gemm_row(bw, prec), n0 = gemm_ncb(bw, prec);
     std::vector<std::pair<int, int>> v{{n0, gemm_ct(n0, bw)}};

@@ -12,6 +12,8 @@
 
 #include "s2_layout.h"
 
+struct s2amd_plan;
+
 namespace s2 {
 
 // ---- error handling -------------------------------------------------------
@@ -120,6 +122,7 @@ struct GemmTables {
     bool n64 = false;      // prec 0: dense FP64 tables for every order (s2_naive64.hip; cut = 0)
     // tile choices from s2amd_plan_autotune (0: the built-in heuristic)
     int t_ncb = 0, t_ct = 0;  // prec 0, 1: data columns per GEMM block, column tiles per table load
+    int t_cols = 0;           // dense FP64: data columns of the calls the choice was timed at and holds for
     int t_gj = 0;             // prec 2: 64-ring groups per inverse GEMM block
     void* af = nullptr;
     void* ai = nullptr;
@@ -226,9 +229,9 @@ void gemm_fwd_launch(const DevConsts& c, const GemmTables& g, const void* Cb, co
                      int F, Fmt fmt, hipStream_t s);
 void gemm_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, void* Cb, void* X,
                      int F, Fmt fmt, hipStream_t s);
-// Tile shapes the GEMMs accept at bw: (columns per block, column tiles per
+// Tile shapes the GEMMs of a call accept: (columns per block, column tiles per
 // table load), the heuristic's choice first.
-std::vector<std::pair<int, int>> gemm_tile_choices(const GemmTables& g);
+std::vector<std::pair<int, int>> gemm_tile_choices(const GemmTables& g, int F, Fmt fmt);
 // 64-ring groups per mixed inverse GEMM block that bw admits, the default first.
 std::vector<int> mix_gj_choices(int bw);
 void gemm_tables_create(GemmTables& g, const DevTables& t, int prec, hipStream_t s);
@@ -237,10 +240,14 @@ void gemm_tables_destroy(GemmTables& g);
 bool n64_supported(int bw, int prec);  // FP64, bw in [16, 512]
 int n64_min_fields(int bw);            // largest call of a plan from which it holds them
 void n64_tables_create(GemmTables& g, const DevTables& t, const DevConsts& c, hipStream_t s);
+int n64_cols(int F, Fmt fmt);  // data columns of a call
+std::vector<std::pair<int, int>> n64_tile_choices(const GemmTables& g, int F, Fmt fmt);
 void n64_fwd_launch(const DevConsts& c, const GemmTables& g, const double2* X, double* cre, double* cim, int F, Fmt fmt,
                     hipStream_t s);
 void n64_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, double2* X, int F,
                     Fmt fmt, hipStream_t s);
+// s2amd_plan_autotune on calls of the given format (that entry point: COMPLEX).
+int plan_autotune(s2amd_plan* p, int nfields, Fmt fmt, hipStream_t s);
 size_t fast_x_bytes(int bw, int prec);   // scratch X per field
 size_t fast_cb_bytes(int bw, int prec);  // scratch Cb per field
 void forward_fast(const DevConsts& c, const GemmTables& g, const double* re, const double* im, double* cre,

@@ -169,7 +169,7 @@ void n64_tables_create(GemmTables& g, const DevTables& t, const DevConsts& c, hi
     S2_HIP(hipStreamSynchronize(s));
 }
 
-static int n64_cols(int F, Fmt fmt) { return (fmt == Fmt::Complex ? 4 : 2) * F; }
+int n64_cols(int F, Fmt fmt) { return (fmt == Fmt::Complex ? 4 : 2) * F; }
 
 // Columns per block of the K-chunked kernels, 0: the direct ones.  Measured,
 // us forward / inverse: direct against 32 columns bw=128 x16 16 / 14, 18 / 17,
@@ -180,6 +180,39 @@ static int n64_cols(int F, Fmt fmt) { return (fmt == Fmt::Complex ? 4 : 2) * F; 
 static int n64_kc_cols(int B, int F) {
     if (B < 128 || (long)F * B * B < 300000) return 0;
     return F >= 64 || (B > 256 && F >= 16) ? 64 : 32;
+}
+// The same for the forward.  bw > 384: its table exceeds the 256 MB memory-side
+// cache, and the direct kernel's waves keep too little of the HBM stream in
+// flight (one field, us, direct / 32 columns: bw=360 55 / 71, bw=400 129 / 85,
+// bw=512 206 / 147; the inverse stays direct, bw=400 65 / 92, bw=512 124 / 120).
+static int n64_fwd_kc_cols(int B, int F) {
+    const int kc = n64_kc_cols(B, F);
+    return kc == 0 && B > 384 ? 32 : kc;
+}
+
+// Column tiles per wave of the direct kernels: the tuned ones for calls of as
+// many data columns as they were timed at, else the rule (its figures beside
+// the launches).
+static int n64_fwd_ct(const GemmTables& g, int cols) {
+    return g.t_cols == cols ? g.t_ct : g.bw > 32 && cols > 512 ? 2 : 1;
+}
+static int n64_inv_ct(const GemmTables& g, int cols) { return g.t_cols == cols ? g.t_ncb / 16 : cols > 256 ? 2 : 1; }
+
+// Choices of a call: (16 x column tiles per wave of the inverse, column tiles
+// of the forward) where a direct kernel serves it, the rule's first.  The
+// K-chunked kernels have nothing to choose: their columns per block, one column
+// tile per wave.
+std::vector<std::pair<int, int>> n64_tile_choices(const GemmTables& g, int F, Fmt fmt) {
+    const int kf = n64_fwd_kc_cols(g.bw, F), ki = n64_kc_cols(g.bw, F);
+    if (kf && ki) return {{ki, 1}};
+    GemmTables rule;
+    rule.bw = g.bw;
+    const int cols = n64_cols(F, fmt), f0 = kf ? 1 : n64_fwd_ct(rule, cols), i0 = n64_inv_ct(rule, cols);
+    std::vector<std::pair<int, int>> v;
+    for (int i : {i0, 3 - i0})
+        for (int f : {f0, 3 - f0})
+            if (f == f0 || !kf) v.push_back({16 * i, f});
+    return v;
 }
 
 template <int CT, int NTW>
@@ -202,19 +235,14 @@ static void n64_inv_direct(const DevConsts& c, const GemmTables& g, const double
 
 void n64_fwd_launch(const DevConsts& c, const GemmTables& g, const double2* X, double* cre, double* cim, int F, Fmt fmt,
                     hipStream_t s) {
-    // bw > 384: the forward table exceeds the 256 MB memory-side cache, and the
-    // direct kernel's waves keep too little of the HBM stream in flight (one field,
-    // us, direct / 32 columns: bw=360 55 / 71, bw=400 129 / 85, bw=512 206 / 147;
-    // the inverse stays direct, bw=400 65 / 92, bw=512 124 / 120)
-    const int B = c.bw, kc = n64_kc_cols(B, F) ? n64_kc_cols(B, F) : B > 384 ? 32 : 0;
+    const int B = c.bw, kc = n64_fwd_kc_cols(B, F);
     if (kc == 64) return (B <= 256 ? n64_fwd_kc_launch<1, 4> : n64_fwd_kc_launch<2, 4>)(c, g, X, cre, cim, F, fmt, s);
     if (kc == 32) return (B <= 256 ? n64_fwd_kc_launch<1, 2> : n64_fwd_kc_launch<2, 2>)(c, g, X, cre, cim, F, fmt, s);
     // tiles per wave: more reuse each load more, fewer give more waves and a
     // shorter stream each (us, column x degree tiles: bw=64 x8 1x1 8.8, 1x2 9.2,
     // x64 13.9, 12.6, x1024 1x2 125, 2x1 114; bw=128 x8 12.0, 14.9; bw=256 x1
     // 23.6, 19.8; bw=300 x1 35, 41; bw=32, one degree tile, x1024 1x1 29, 2x1 32)
-    const int ct = g.t_ct ? g.t_ct : B > 32 && n64_cols(F, fmt) > 512 ? 2 : 1;
-    if (ct == 2) n64_fwd_direct<2, 1>(c, g, X, cre, cim, F, fmt, s);
+    if (n64_fwd_ct(g, n64_cols(F, fmt)) == 2) n64_fwd_direct<2, 1>(c, g, X, cre, cim, F, fmt, s);
     else if (B > 32 && (F >= 16 || (B >= 192 && B <= 288))) n64_fwd_direct<1, 2>(c, g, X, cre, cim, F, fmt, s);
     else n64_fwd_direct<1, 1>(c, g, X, cre, cim, F, fmt, s);
 }
@@ -244,8 +272,7 @@ void n64_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, 
     }
     // as in the forward (us, column x ring tiles: bw=64 x8 1x1 7.9, 1x2 8.7, x64
     // 13.7, 11.4, x1024 1x2 115, 2x2 99; bw=128 x8 13.4, 10.6; bw=256 x1 18.3, 17.1)
-    const int ct = g.t_ct ? g.t_ct : n64_cols(F, fmt) > 256 ? 2 : 1;
-    if (ct == 2) n64_inv_direct<2, 2>(c, g, cre, cim, X, F, fmt, s);
+    if (n64_inv_ct(g, n64_cols(F, fmt)) == 2) n64_inv_direct<2, 2>(c, g, cre, cim, X, F, fmt, s);
     else if (B >= 192 || F * B >= 1024) n64_inv_direct<1, 2>(c, g, cre, cim, X, F, fmt, s);
     else n64_inv_direct<1, 1>(c, g, cre, cim, X, F, fmt, s);
 }

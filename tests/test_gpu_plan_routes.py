@@ -64,3 +64,24 @@ def test_convolutions_do_not_depend_on_the_field_count(env, bw):
         for f in range(F):
             plan.conv(*[v[f:f + 1] for v in t], x[f:f + 1], y[f:f + 1])
     assert torch.equal(a, x) and torch.equal(b, y)
+
+
+@pytest.mark.parametrize("bw,F,want", [
+    (256, 8, {(32, 1)}), (256, 64, {(64, 1)}), (300, 16, {(64, 1)}), (512, 4, {(32, 1)}),  # K-chunked: one shape
+    (512, 1, {(16, 1), (32, 1)}),  # K-chunked forward, direct inverse
+    (64, 3, {(16, 1), (16, 2), (32, 1), (32, 2)}), (64, 80, {(16, 1), (16, 2), (32, 1), (32, 2)})])
+def test_autotune_of_dense_plans(env, bw, F, want):
+    # The choice reported is one that the call runs, and calls of every size
+    # keep their bits.
+    S, torch, dev = env
+    print(f"autotune bw={bw} F={F}", flush=True)
+    top = max(F, 4)
+    g, h = grids(torch, dev, bw, top, bw + F)
+    with contextlib.closing(S.Plan(bw, top)) as plan:
+        before = {(k, fmt): pair(torch, plan, g[:k], h[:k], fmt) for k in {1, F, top} for fmt in (0, 1)}
+        assert plan.tuning() == (0, 0, 0)
+        plan.autotune(F)
+        cols, tiles, rings = plan.tuning()
+        assert (cols, tiles) in want and rings == 0
+        for (k, fmt), outs in before.items():
+            assert all(torch.equal(u, v) for u, v in zip(pair(torch, plan, g[:k], h[:k], fmt), outs)), (k, fmt)
