@@ -332,7 +332,7 @@ __device__ __forceinline__ void naive64_fwd_block(const double2* __restrict__ X,
         case 7: naive64_fwd_kc<7, H, CT>(X, NF, g, cre, cim, m, cb, B, F, fmt, sm); break;
         case 8: naive64_fwd_kc<8, H, CT>(X, NF, g, cre, cim, m, cb, B, F, fmt, sm); break;
         case 9: naive64_fwd_kc<9, H, CT>(X, NF, g, cre, cim, m, cb, B, F, fmt, sm); break;
-        default: break;  // none (n64_kc_supported)
+        default: break;  // none (refused by n64_fwd_kc_launch)
     }
 }
 
@@ -375,7 +375,12 @@ void n64_fwd_kc_launch(const DevConsts& c, const GemmTables& g, const double2* X
                        Fmt fmt, hipStream_t s) {
     const int B = c.bw, nb = ((fmt == Fmt::Complex ? 4 : 2) * F + 16 * CT - 1) / (16 * CT);
     int nt = 0;
-    for (int q = 0; q < mix_npairs(B); ++q) nt = std::max(nt, n64_nt(q, B));
+    for (int q = 0; q < mix_npairs(B); ++q) {
+        const int n = n64_nt(q, B);
+        // the instances of naive64_fwd_block: 5 to 9 tiles per wave (every bw in [128, 512])
+        if (n < 5 * H || n > 9 * H) throw ArgError{"dense FP64 forward: no K-chunked kernel at this bandwidth"};
+        nt = std::max(nt, n);
+    }
     const dim3 grid(mix_npairs8(B) * nb);
     const size_t lds = sizeof(double) * n64_fwd_lds(nt, CT);
     const double* nf = (const double*)g.af;
