@@ -85,3 +85,51 @@ def test_autotune_of_dense_plans(env, bw, F, want):
         assert (cols, tiles) in want and rings == 0
         for (k, fmt), outs in before.items():
             assert all(torch.equal(u, v) for u, v in zip(pair(torch, plan, g[:k], h[:k], fmt), outs)), (k, fmt)
+
+
+@pytest.mark.parametrize("bw,F,prec,cutoff", [
+    (8, 2, 0, 8), (8, 2, 0, 3), (11, 3, 0, 11), (64, 1, 0, 64), (64, 9, 0, 64), (100, 5, 0, 100), (131, 2, 0, 131),
+    (128, 65, 0, 128), (512, 1, 0, 512), (512, 3, 0, 200), (600, 1, 0, 100), (600, 2, 0, 600), (128, 65, 1, 128),
+    (64, 5, 1, 20), (32, 3, 2, 32), (100, 5, 2, 100), (131, 2, 2, 131), (128, 65, 2, 128), (64, 9, 3, 64)])
+def test_real_calls_read_no_stale_row(env, bw, F, prec, cutoff):
+    # REAL calls neither write nor read the order rows m >= bw of the
+    # intermediate, in every ring FFT and Legendre instance: NaN left there by a
+    # COMPLEX call does not reach them.
+    S, torch, dev = env
+    print(f"stale rows bw={bw} F={F} prec={prec} cutoff={cutoff}", flush=True)
+    g, h = grids(torch, dev, bw, F, bw)
+    bad = torch.full_like(g, float("nan"))
+    out = []
+    for poison in (False, True):
+        with contextlib.closing(S.Plan(bw, F, precision=prec, cutoff=cutoff)) as plan:
+            a, b = (torch.empty((F, bw * bw), dtype=torch.float64, device=dev) for _ in range(2))
+            x, y = torch.empty_like(g), torch.empty_like(g)
+            if poison:
+                pair(torch, plan, bad, bad, 0)
+            plan.forward(g, h, a, b, data_format=1)
+            if poison:
+                pair(torch, plan, bad, bad, 0)
+            plan.inverse(a, b, x, y, data_format=1)
+            out.append((a, b, x, y))
+    for u, v in zip(*out):
+        assert bool(torch.isfinite(v).all()) and torch.equal(u, v)
+
+
+@pytest.mark.parametrize("bw,F,prec", [(64, 481, 2), (200, 129, 2), (255, 97, 2), (64, 481, 3), (128, 225, 3)])
+def test_real_pair_workgroups_match_order_workgroups(env, bw, F, prec):
+    # Mixed and split REAL calls on both sides of the line between workgroups of
+    # one order (fewer than 512 order-pair workgroups) and of order pairs.
+    S, torch, dev = env
+    pairs = ((bw + 1) // 2 + 7) // 8 * 8
+
+    def workgroups(n):  # of the forward; 64 data columns each, two per REAL field
+        return pairs * -(-2 * n // 64)
+
+    assert workgroups(F) >= 512 > workgroups(3)
+    print(f"REAL pair workgroups bw={bw} F={F} prec={prec}", flush=True)
+    g, h = grids(torch, dev, bw, F, bw + F)
+    with contextlib.closing(S.Plan(bw, F, precision=prec)) as plan:
+        whole = pair(torch, plan, g, h, 1)
+        for f in (0, F - 3):
+            for u, v in zip(pair(torch, plan, g[f:f + 3], h[f:f + 3], 1), whole):
+                assert torch.equal(u, v[f:f + 3])
