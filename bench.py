@@ -138,18 +138,21 @@ def kernel_map(form, bw, nfields):
     block; 512 threads up to bw = 256, 1024 above) at bw in [128, 512] with 64
     or more fields; so do the dense FP64 ones (the inverse always 512
     threads), above bw = 256 from 16 fields, and with 32 columns per block
-    (negative last argument in the forward) from bw^2 x fields = 300000."""
+    (negative last argument in the forward) from bw^2 x fields = 300000, but
+    for four fields or fewer, whose 16 columns are one tile."""
     k = dict(KERNELS[form] if bw & (bw - 1) == 0 else kernels_gen(bw, form))
     if dense_fp64(form, bw, nfields):
         k.pop("dct_fwd"), k.pop("dct_inv")
         h = 1 if bw <= 256 else 2
-        if bw >= 128 and nfields * bw * bw >= 300000:
-            if nfields >= 64 or (h == 2 and nfields >= 16):
-                k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd_kc<double, {512 * h}>", "k_gemm_inv_kc<double, 512>"
-            else:
-                k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd<double, false, 2, {-h}>", "k_gemm_inv_kc<double, 256>"
+        k["leg_fwd"], k["leg_inv"] = "k_gemm_fwd<double, false, CT", "k_gemm_inv<double, false, CT"
+        many = bw >= 128 and nfields * bw * bw >= 300000
+        if many and (nfields >= 64 or (h == 2 and nfields >= 16)):
+            k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd_kc<double, {512 * h}>", "k_gemm_inv_kc<double, 512>"
         else:
-            k["leg_fwd"], k["leg_inv"] = "k_gemm_fwd<double, false, CT", "k_gemm_inv<double, false, CT"
+            if bw > 384 or many and (nfields > 4 or 4 * nfields * bw * bw >= 1600000):
+                k["leg_fwd"] = f"k_gemm_fwd<double, false, 2, {-h}>"
+            if many and (nfields > 4 or bw >= 480):
+                k["leg_inv"] = "k_gemm_inv_kc<double, 256>"
     elif form == "fp32" and 128 <= bw <= 512 and nfields >= 64:
         t = 512 if bw <= 256 else 1024
         k["leg_fwd"], k["leg_inv"] = f"k_gemm_fwd_kc<float, {t}>", f"k_gemm_inv_kc<float, {t}>"

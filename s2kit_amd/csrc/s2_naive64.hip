@@ -123,7 +123,7 @@ bool n64_supported(int bw, int prec) { return prec == 0 && bw >= 16 && bw <= 512
 // 77 / 69 against 63 / 64, x4 82 / 75 against 87 / 88, bw=512 x2 143 / 110
 // against 104 / 98, x4 152 / 118 against 144 / 128, x8 173 / 131 against
 // 217 / 210).  A plan holds one kind and runs its smaller calls on it as well
-// (one field, dense against seminaive: bw=400 85 / 65 against 58 / 57, bw=512
+// (one field, dense against seminaive: bw=400 85 / 64 against 58 / 57, bw=512
 // 147 / 124 against 72 / 80): with both, a field's last bits depended on its
 // call's field count, and a plan held two table sets (bw=512 x8 2201 -> 1670 MB).
 int n64_min_fields(int bw) { return bw <= 320 ? 1 : 4; }
@@ -176,19 +176,27 @@ int n64_cols(int F, Fmt fmt) { return (fmt == Fmt::Complex ? 4 : 2) * F; }
 // x32 26 / 19, 22 / 18; bw=256 x4 24 / 20, 34 / 23, x8 37 / 25, 38 / 24, x16
 // 72 / 46, 45 / 39; bw=300 x4 46 / 32, 47 / 33; 32 against 64 columns bw=256 x8
 // 38 / 24, 52 / 31, x32 63 / 65, 63 / 59; bw=512 x8 173 / 131, 185 / 168, x16
-// 257 / 192, 233 / 187.  (bw = 100 x128 direct: 44 / 40.)
+// 257 / 192, 233 / 187.  (bw = 100 x128 direct: 44 / 40.)  These are COMPLEX
+// calls; REAL ones, of half the columns, follow the same lines in fields.
 static int n64_kc_cols(int B, int F) {
     if (B < 128 || (long)F * B * B < 300000) return 0;
     return F >= 64 || (B > 256 && F >= 16) ? 64 : 32;
 }
-// The same for the forward.  bw > 384: its table exceeds the 256 MB memory-side
+// A call of one column tile (at most 16 columns, whatever the format) fills half
+// of a 32-column block: the direct kernels are faster, in the forward until the
+// table stream outgrows them, by columns x bw^2, and in the inverse to bw = 480
+// (whole calls, us, 32 columns / direct: forward, REAL, bw=256 x8 48.5 / 37.8,
+// bw=320 x4 60.7 / 53.5, bw=340 x7 87.6 / 90.3, COMPLEX bw=300 x4 62.4 / 56.1,
+// bw=352 x4 80.9 / 81.7; inverse, COMPLEX, bw=321 x4 73 / 62, bw=400 x4 117 / 105,
+// bw=448 x4 136 / 133, bw=500 x4 171 / 175, bw=512 x4 181 / 196, REAL bw=400 x4
+// 111 / 94).  Past bw = 384 the forward's table exceeds the 256 MB memory-side
 // cache, and the direct kernel's waves keep too little of the HBM stream in
-// flight (one field, us, direct / 32 columns: bw=360 55 / 71, bw=400 129 / 85,
-// bw=512 206 / 147; the inverse stays direct, bw=400 65 / 92, bw=512 124 / 120).
-static int n64_fwd_kc_cols(int B, int F) {
-    const int kc = n64_kc_cols(B, F);
-    return kc == 0 && B > 384 ? 32 : kc;
+// flight (one field: bw=360 71 / 55, bw=400 85 / 129, bw=512 147 / 206).
+static int n64_fwd_kc_cols(int B, int F, int cols) {
+    if (B > 384) return std::max(32, n64_kc_cols(B, F));
+    return cols <= 16 && (long)cols * B * B < 1600000 ? 0 : n64_kc_cols(B, F);
 }
+static int n64_inv_kc_cols(int B, int F, int cols) { return cols <= 16 && B < 480 ? 0 : n64_kc_cols(B, F); }
 
 // Column tiles per wave of the direct kernels: the tuned ones for calls of as
 // many data columns as they were timed at, else the rule (its figures beside
@@ -203,15 +211,15 @@ static int n64_inv_ct(const GemmTables& g, int cols) { return g.t_cols == cols ?
 // K-chunked kernels have nothing to choose: their columns per block, one column
 // tile per wave.
 std::vector<std::pair<int, int>> n64_tile_choices(const GemmTables& g, int F, Fmt fmt) {
-    const int kf = n64_fwd_kc_cols(g.bw, F), ki = n64_kc_cols(g.bw, F);
+    const int cols = n64_cols(F, fmt), kf = n64_fwd_kc_cols(g.bw, F, cols), ki = n64_inv_kc_cols(g.bw, F, cols);
     if (kf && ki) return {{ki, 1}};
     GemmTables rule;
     rule.bw = g.bw;
-    const int cols = n64_cols(F, fmt), f0 = kf ? 1 : n64_fwd_ct(rule, cols), i0 = n64_inv_ct(rule, cols);
+    const int f0 = kf ? 1 : n64_fwd_ct(rule, cols), i0 = n64_inv_ct(rule, cols);
     std::vector<std::pair<int, int>> v;
     for (int i : {i0, 3 - i0})
         for (int f : {f0, 3 - f0})
-            if (f == f0 || !kf) v.push_back({16 * i, f});
+            if ((f == f0 || !kf) && (i == i0 || !ki)) v.push_back({16 * i, f});
     return v;
 }
 
@@ -235,15 +243,19 @@ static void n64_inv_direct(const DevConsts& c, const GemmTables& g, const double
 
 void n64_fwd_launch(const DevConsts& c, const GemmTables& g, const double2* X, double* cre, double* cim, int F, Fmt fmt,
                     hipStream_t s) {
-    const int B = c.bw, kc = n64_fwd_kc_cols(B, F);
+    const int B = c.bw, cols = n64_cols(F, fmt), kc = n64_fwd_kc_cols(B, F, cols);
     if (kc == 64) return (B <= 256 ? n64_fwd_kc_launch<1, 4> : n64_fwd_kc_launch<2, 4>)(c, g, X, cre, cim, F, fmt, s);
     if (kc == 32) return (B <= 256 ? n64_fwd_kc_launch<1, 2> : n64_fwd_kc_launch<2, 2>)(c, g, X, cre, cim, F, fmt, s);
     // tiles per wave: more reuse each load more, fewer give more waves and a
     // shorter stream each (us, column x degree tiles: bw=64 x8 1x1 8.8, 1x2 9.2,
     // x64 13.9, 12.6, x1024 1x2 125, 2x1 114; bw=128 x8 12.0, 14.9; bw=256 x1
-    // 23.6, 19.8; bw=300 x1 35, 41; bw=32, one degree tile, x1024 1x1 29, 2x1 32)
-    if (n64_fwd_ct(g, n64_cols(F, fmt)) == 2) n64_fwd_direct<2, 1>(c, g, X, cre, cim, F, fmt, s);
-    else if (B > 32 && (F >= 16 || (B >= 192 && B <= 288))) n64_fwd_direct<1, 2>(c, g, X, cre, cim, F, fmt, s);
+    // 23.6, 19.8; bw=300 x1 35, 41; bw=32, one degree tile, x1024 1x1 29, 2x1 32).
+    // Few fields at bw 192 to 256: order 0's six to eight degree tiles in pairs fit
+    // one block of four waves, from nine on they need a second, nearly empty one
+    // (whole calls, one field, 1x1 / 1x2: bw=192 26.4 / 23.6, bw=200 28.7 / 26.6,
+    // bw=256 29.4 / 25.8, bw=257 34 / 43, bw=272 34 / 43, bw=288 41 / 46)
+    if (n64_fwd_ct(g, cols) == 2) n64_fwd_direct<2, 1>(c, g, X, cre, cim, F, fmt, s);
+    else if (B > 32 && (F >= 16 || (B >= 192 && B <= 256))) n64_fwd_direct<1, 2>(c, g, X, cre, cim, F, fmt, s);
     else n64_fwd_direct<1, 1>(c, g, X, cre, cim, F, fmt, s);
 }
 
@@ -260,9 +272,9 @@ static void n64_inv_split(int B, int& jt, int& nz) {
 
 void n64_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, const double* cim, double2* X, int F,
                     Fmt fmt, hipStream_t s) {
-    const int B = c.bw, kc = n64_kc_cols(B, F);
+    const int B = c.bw, cols = n64_cols(F, fmt), kc = n64_inv_kc_cols(B, F, cols);
     if (kc) {
-        const int nb = (n64_cols(F, fmt) + kc - 1) / kc;
+        const int nb = (cols + kc - 1) / kc;
         int jt = 1, nz = 1;
         n64_inv_split(B, jt, nz);
         launch_lds(kc == 64 ? k_gemm_inv_kc<double, 512> : k_gemm_inv_kc<double, 256>, dim3(mix_npairs8(B) * nb * nz),
@@ -272,7 +284,7 @@ void n64_inv_launch(const DevConsts& c, const GemmTables& g, const double* cre, 
     }
     // as in the forward (us, column x ring tiles: bw=64 x8 1x1 7.9, 1x2 8.7, x64
     // 13.7, 11.4, x1024 1x2 115, 2x2 99; bw=128 x8 13.4, 10.6; bw=256 x1 18.3, 17.1)
-    if (n64_inv_ct(g, n64_cols(F, fmt)) == 2) n64_inv_direct<2, 2>(c, g, cre, cim, X, F, fmt, s);
+    if (n64_inv_ct(g, cols) == 2) n64_inv_direct<2, 2>(c, g, cre, cim, X, F, fmt, s);
     else if (B >= 192 || F * B >= 1024) n64_inv_direct<1, 2>(c, g, cre, cim, X, F, fmt, s);
     else n64_inv_direct<1, 1>(c, g, cre, cim, X, F, fmt, s);
 }

@@ -133,3 +133,20 @@ def test_real_pair_workgroups_match_order_workgroups(env, bw, F, prec):
         for f in (0, F - 3):
             for u, v in zip(pair(torch, plan, g[f:f + 3], h[f:f + 3], 1), whole):
                 assert torch.equal(u, v[f:f + 3])
+
+
+@pytest.mark.parametrize("bw,F,k,fmt", [
+    (194, 9, 8, 1), (256, 9, 8, 1), (257, 5, 4, 0), (274, 5, 4, 0), (316, 5, 4, 0), (317, 5, 4, 0), (340, 9, 7, 1),
+    (384, 9, 5, 1), (385, 5, 4, 0), (447, 9, 8, 1), (479, 5, 4, 0), (480, 5, 4, 0)])
+def test_calls_of_one_column_tile(env, bw, F, k, fmt):
+    # Calls of at most 16 data columns run the direct dense kernels where larger
+    # ones run K-chunked (forward and inverse to lines of their own): the same bits.
+    S, torch, dev = env
+    print(f"one column tile bw={bw} F={F} k={k} fmt={fmt}", flush=True)
+    g, h = grids(torch, dev, bw, F, bw)
+    assert k * (2 if fmt else 4) <= 16 < F * (2 if fmt else 4)
+    with contextlib.closing(S.Plan(bw, F)) as plan:
+        whole = pair(torch, plan, g, h, fmt)
+        for f in (0, F - k):
+            for u, v in zip(pair(torch, plan, g[f:f + k], h[f:f + k], fmt), whole):
+                assert torch.equal(u, v[f:f + k]), f
