@@ -119,7 +119,8 @@ int s2amd_inverse(s2amd_plan* plan, const double* cre, const double* cim, double
 #define S2AMD_NOALLOC_SCRATCH_BYTES ((size_t)128 << 20)
 int s2amd_forward_noalloc(s2amd_plan* plan, const double* re, const double* im, double* cre, double* cim,
                           int nfields, int data_format, void* stream);
-/* Zonal coefficients zr/zi [nfields][bw] (FZTSemiMemo per field). */
+/* Zonal coefficients zr/zi [nfields][bw] (FZTSemiMemo per field); the plan's
+ * cutoff must be 1 or more (S2AMD_EINVAL else: order 0 has no cosine table). */
 int s2amd_zonal(s2amd_plan* plan, const double* re, const double* im, double* zr, double* zi, int nfields,
                 int data_format, void* stream);
 /* ConvOn2SphereSemiMemo per field: signal s, filter h (grids), output o. */

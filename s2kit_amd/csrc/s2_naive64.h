@@ -13,8 +13,8 @@
 // the multiplications but needs a DCT pass over the order rows each way
 // (24 N^2 bytes per field at the HBM rate), and its staircase tables left the
 // matrix cores mostly waiting.  bw=256 x 1024 fields, DCT + seminaive GEMM
-// against one dense GEMM: forward 1.46 + 1.36 -> 1.52 ms, inverse 1.16 + 1.55
-// -> 1.72 ms (step 8.28 -> 6.07 ms); bw=512 x 128 2.0 -> 1.41, 1.7 -> 1.39 ms;
+// against one dense GEMM: forward 1.46 + 1.36 -> 1.57 ms, inverse 1.16 + 1.55
+// -> 1.75 ms (step 8.28 -> 6.19 ms); bw=512 x 128 2.0 -> 1.41, 1.7 -> 1.39 ms;
 // bw=64 x1 16 -> 7, 17 -> 6 us.  The dense sums have no cosine-space
 // cancellation: error against 64-bit definitions 4.1e-14 -> 1.4e-14.
 //

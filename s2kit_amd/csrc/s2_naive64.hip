@@ -111,8 +111,8 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4))) void k
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// At bw = 512 the tables take 0.54 GB per direction; at 1024 they would take
-// 4.3 GB, which the few fields that fit beside them could not stream as fast
+// At bw = 512 the tables take 0.60 GB (forward) and 0.55 GB; at 1024 they would
+// take over 4.3 GB each, which the few fields that fit beside them could not stream as fast
 // as the seminaive tables' 1.4 GB.
 bool n64_supported(int bw, int prec) { return prec == 0 && bw >= 16 && bw <= 512; }
 

@@ -13,14 +13,15 @@ namespace s2 {
 // ---------------------------------------------------------------------------
 // A block runs an order pair (m, bw-1-m) (about bw+1 degrees, so blocks are
 // alike) for 64 data columns (CT = 4 column tiles), or 32 (CT = 2) for calls of
-// fewer than 64 fields.  Table stages go global -> LDS by DMA, the data
+// fewer than 64 fields (above bw = 256, 16).  Table stages go global -> LDS by DMA, the data
 // through registers (folded, in the forward) into LDS, both in MFMA operand
 // order: every LDS read is 64 consecutive doubles.  An FP64 16x16x4 MFMA
 // holds its SIMD's matrix core for 64 cycles and needs one 512-byte operand
 // read, a quarter of the LDS rate with all four SIMDs busy, so the kernel is
 // bound by the matrix cores once four waves per SIMD cover the stages'
-// latency (bw=256 x 1024 forward: matrix cores busy 70% of 1.52 ms, 5.8 GB of HBM
-// traffic at 3.8 TB/s; 45-50 of 71.9 TF/s that a large library product reaches);
+// latency (bw=256 x 1024 forward: matrix cores busy 70% of 1.57 ms, 5.8 GB of HBM
+// traffic at 3.7 TB/s; 44 TF/s, 49 with the padding, of 71.9 that a large library
+// product reaches);
 // hence 128 VGPRs, two stage buffers within 80 KiB of LDS and (CT = 4,
 // bw <= 256) two blocks per CU.
 //

@@ -150,3 +150,12 @@ def test_calls_of_one_column_tile(env, bw, F, k, fmt):
         for f in (0, F - k):
             for u, v in zip(pair(torch, plan, g[f:f + k], h[f:f + k], fmt), whole):
                 assert torch.equal(u, v[f:f + k]), f
+
+
+def test_zonal_needs_a_seminaive_order(env):
+    S, torch, dev = env
+    g, h = grids(torch, dev, 16, 2, 1)
+    z = [torch.empty((2, 16), dtype=torch.float64, device=dev) for _ in range(2)]
+    with contextlib.closing(S.Plan(16, 2, cutoff=0)) as plan:
+        with pytest.raises(S.S2Error, match="cosine table"):
+            plan.zonal(g, h, *z)
